@@ -293,7 +293,9 @@ def _decode_inputs(case, seed):
 
 
 def prepare(case, seed):
-    return {"encode": _Encoder, "matmul": _Product, "dequant": _Decode}[case["path"]](case, seed)
+    state = {"encode": _Encoder, "matmul": _Product, "dequant": _Decode}[case["path"]](case, seed)
+    torch.cuda.synchronize()  # inputs are made on another stream than the passes run on
+    return state
 
 
 def run(state):
