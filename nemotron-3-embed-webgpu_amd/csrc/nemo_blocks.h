@@ -208,17 +208,14 @@ __device__ __forceinline__ void q40_expand(const Q40Fetch& f, half8v* lo, half8v
   hi[1] = to_half8(vh + 8);
 }
 
-// Q4_K raw: 8 threads per 144-byte block. Thread c writes output chunks c,
-// c + 8, c + 16, c + 24 of 8 values (values 64 i + 8 c .. +8 for group i),
-// so each store instruction of 8 neighbouring lanes fills 128 contiguous
-// bytes (f16) or 256 (f32): the low nibbles of bytes 8c .. 8c + 8 of every
-// group's 32 (c < 4) or the high nibbles of bytes 8(c - 4) .. (c >= 4).
+// Q4_K raw -> f16: 8 threads per 144-byte block. Thread c (0..7) of the block
+// at `blk` writes output chunks c, c + 8, c + 16, c + 24 of 8 values (values
+// 64 i + 8 c .. +8 for group i), so each store instruction of 8 neighbouring
+// lanes fills 128 contiguous bytes: the low nibbles of bytes 8c .. 8c + 8 of
+// every group's 32 (c < 4) or the high nibbles of bytes 8(c - 4) .. (c >= 4).
 // NT: non-temporal stores, for output that is not read back soon.
-// Thread c (0..7) of the 144-byte block at `blk`, whose values start at
-// element o of the outputs.
 template <bool NT>
-__device__ __forceinline__ void q4k_block_part(const uint8_t* __restrict__ blk, int c, int64_t o0,
-                                               float* __restrict__ out32, uint16_t* __restrict__ out16) {
+__device__ __forceinline__ void q4k_block_part(const uint8_t* __restrict__ blk, int c, uint16_t* __restrict__ out) {
   const int part = c & 3, high = c >> 2;
   const u32x4 hdr = *(const u32x4*)blk;
   uint32_t q[4][2];
@@ -237,20 +234,9 @@ __device__ __forceinline__ void q4k_block_part(const uint8_t* __restrict__ blk, 
     float v[8];
     nibbles4_fma((q[i][0] >> sh) & 0x0f0f0f0fu, dsc, ndm, v);
     nibbles4_fma((q[i][1] >> sh) & 0x0f0f0f0fu, dsc, ndm, v + 4);
-    const int64_t o = o0 + 64 * i + 8 * c;
-    if constexpr (NT) {
-      if (out32) {
-        __builtin_nontemporal_store(float4v{v[0], v[1], v[2], v[3]}, (float4v*)(out32 + o));
-        __builtin_nontemporal_store(float4v{v[4], v[5], v[6], v[7]}, (float4v*)(out32 + o + 4));
-      }
-      if (out16) __builtin_nontemporal_store(to_half8(v), (half8v*)(out16 + o));
-    } else {
-      if (out32) {
-        *(float4v*)(out32 + o) = float4v{v[0], v[1], v[2], v[3]};
-        *(float4v*)(out32 + o + 4) = float4v{v[4], v[5], v[6], v[7]};
-      }
-      if (out16) *(half8v*)(out16 + o) = to_half8(v);
-    }
+    half8v* o = (half8v*)(out + 64 * i + 8 * c);
+    if constexpr (NT) __builtin_nontemporal_store(to_half8(v), o);
+    else *o = to_half8(v);
   }
 }
 
@@ -300,7 +286,7 @@ __device__ __forceinline__ void side_expand_part(const SideExpand& e, int64_t b,
   const uint8_t* blocks = second ? e.part[1].blocks : e.part[0].blocks;
   uint16_t* out = second ? e.part[1].out : e.part[0].out;
   if (type == kQ4_K) {
-    q4k_block_part<false>(blocks + b * 144, c, b * 256, nullptr, out);
+    q4k_block_part<false>(blocks + b * 144, c, out + b * 256);
   } else {
     const uint16_t* d = second ? e.part[1].d : e.part[0].d;
     q6k_block_part(blocks + b * 208, d[b], c, out + b * 256);

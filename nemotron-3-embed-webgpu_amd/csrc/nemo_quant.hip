@@ -549,13 +549,14 @@ hipError_t launch_gemv(const uint16_t* x, int ldx, const QWeight& w, uint16_t* y
 // Standalone decoding.
 // ---------------------------------------------------------------------------
 
+// Q4_K -> f16 (the two-pass GEMM's first pass, and standalone with NT).
 template <bool NT>
 __global__ __launch_bounds__(256) void dequant_q4k_kernel(const uint8_t* __restrict__ raw, int64_t n_blocks,
-                                                          float* __restrict__ out32, uint16_t* __restrict__ out16) {
+                                                          uint16_t* __restrict__ out16) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t b = t >> 3;
   if (b >= n_blocks) return;
-  q4k_block_part<NT>(raw + b * 144, (int)(t & 7), b * 256, out32, out16);
+  q4k_block_part<NT>(raw + b * 144, (int)(t & 7), out16 + b * 256);
 }
 
 // Two matrices in one launch: blocks [0, n0) of raw0 to out0, then the n1 of
@@ -567,9 +568,9 @@ __global__ __launch_bounds__(256) void expand_q4k_pair_kernel(const uint8_t* __r
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t b = t >> 3;
   if (b < n0) {
-    q4k_block_part<false>(raw0 + b * 144, (int)(t & 7), b * 256, nullptr, out0);
+    q4k_block_part<false>(raw0 + b * 144, (int)(t & 7), out0 + b * 256);
   } else if ((b -= n0) < n1) {
-    q4k_block_part<false>(raw1 + b * 144, (int)(t & 7), b * 256, nullptr, out1);
+    q4k_block_part<false>(raw1 + b * 144, (int)(t & 7), out1 + b * 256);
   }
 }
 
@@ -583,16 +584,52 @@ hipError_t launch_expand_q4k_pair(const uint8_t* blocks0, int64_t n0, uint16_t* 
 
 hipError_t launch_expand_q4k(const uint8_t* blocks, int64_t n_blocks, uint16_t* out16, hipStream_t stream) {
   if (n_blocks <= 0) return hipSuccess;
-  dequant_q4k_kernel<false><<<(unsigned)((n_blocks * 8 + 255) / 256), 256, 0, stream>>>(blocks, n_blocks, nullptr,
-                                                                                        out16);
+  dequant_q4k_kernel<false><<<(unsigned)((n_blocks * 8 + 255) / 256), 256, 0, stream>>>(blocks, n_blocks, out16);
   return hipGetLastError();
+}
+
+// Standalone decoding is bound by HBM, and by its stores as much as its
+// loads: a store instruction whose lanes leave gaps writes half lines. So each
+// output has the mapping that fills whole lines. float32 (and float32 + f16):
+// thread c of 8 takes values 32 j + 4 c .. +4 of a 256-value block, j = 0..7,
+// so 8 neighbouring lanes store 128 contiguous bytes; f16 alone: values
+// 64 j + 8 c .. +8, the same 128 bytes. 256 M values, us before and after:
+// Q4_K f32 432 -> 192, Q6_K f32 318 -> 179, Q6_K f16 185 -> 104, Q4_0 f32
+// 257 -> 184, Q4_0 f16 149 -> 93 (Q4_K f16 had it: 93): 6.1-7.0 TB/s.
+__device__ __forceinline__ void store_values4(float4v v, int64_t o, float* __restrict__ out32,
+                                              uint16_t* __restrict__ out16) {
+  __builtin_nontemporal_store(v, (float4v*)(out32 + o));
+  if (out16) __builtin_nontemporal_store(__builtin_convertvector(v, half4v), (half4v*)(out16 + o));
+}
+
+__global__ __launch_bounds__(256) void dequant_q4k_f32_kernel(const uint8_t* __restrict__ raw, int64_t n_blocks,
+                                                              float* __restrict__ out32, uint16_t* __restrict__ out16) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t b = t >> 3;
+  if (b >= n_blocks) return;
+  const int c = (int)(t & 7);
+  const uint8_t* blk = raw + b * 144;
+  const u32x4 hdr = *(const u32x4*)blk;
+  uint32_t q[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q[i] = *(const uint32_t*)(blk + 16 + 32 * i + 4 * c);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float dsc0, ndm0, dsc1, ndm1, v[8];
+    q4k_group_factors(hdr, i, dsc0, ndm0, dsc1, ndm1);
+    nibbles4_fma(q[i] & 0x0f0f0f0fu, dsc0, ndm0, v);
+    nibbles4_fma((q[i] >> 4) & 0x0f0f0f0fu, dsc1, ndm1, v + 4);
+    const int64_t o = b * 256 + 64 * i + 4 * c;
+    store_values4(float4v{v[0], v[1], v[2], v[3]}, o, out32, out16);
+    store_values4(float4v{v[4], v[5], v[6], v[7]}, o + 32, out32, out16);
+  }
 }
 
 // Blocks whose size is not a multiple of 16 bytes (Q6_K 210, Q4_0 18) are
 // staged: a workgroup copies a span of whole blocks, which starts 16-byte
 // aligned, from HBM into LDS with 16-byte loads, then decodes from LDS.
-constexpr int kQ6Span = 32;   // 32 * 210 = 6720 bytes = 420 * 16
-constexpr int kQ40Span = 64;  // 64 * 18 = 1152 bytes = 72 * 16
+constexpr int kQ6Span = 32;    // 32 * 210 = 6720 bytes = 420 * 16
+constexpr int kQ40Span = 256;  // 256 * 18 = 4608 bytes = 288 * 16
 
 __device__ __forceinline__ void stage_span(const uint8_t* __restrict__ src, int bytes, uint8_t* lds) {
   const int vec = bytes >> 4;
@@ -603,76 +640,115 @@ __device__ __forceinline__ void stage_span(const uint8_t* __restrict__ src, int 
   __syncthreads();
 }
 
-// Q6_K raw: thread t decodes 32 values (half c/4, quadrant c%4, lanes 0..31)
-// of block t/8 of the span (src/gguf/quantization.ts:53-71).
+// The 4 bytes at any byte offset of a 4-byte aligned LDS array (the word past
+// the last one is read too, and its bytes dropped).
+__device__ __forceinline__ uint32_t lds_word(const uint8_t* lds, int offset) {
+  const uint32_t* w = (const uint32_t*)lds + (offset >> 2);
+  return __builtin_amdgcn_alignbyte(w[1], w[0], (uint32_t)(offset & 3));
+}
+
+// Four values of quadrant Q from their ql and qh bytes: dsc * (q - 32), the
+// product of the reference (the sign of its zeros too).
+__device__ __forceinline__ float4v q6k_values4(uint32_t ql, uint32_t qh, int Q, float dsc) {
+  const uint32_t q = opaque(((ql >> (Q >= 2 ? 4 : 0)) & 0x0f0f0f0fu) | (((qh >> (2 * Q)) & 0x03030303u) << 4));
+  return float4v{dsc * ((float)(q & 0xffu) - 32.0f), dsc * ((float)((q >> 8) & 0xffu) - 32.0f),
+                 dsc * ((float)((q >> 16) & 0xffu) - 32.0f), dsc * ((float)(q >> 24) - 32.0f)};
+}
+
+// Q6_K raw (src/gguf/quantization.ts:53-71): value 128 h + 32 Q + l of a block
+// takes its low bits from ql[64 h + 32 (Q & 1) + l] (high nibble for Q >= 2),
+// its high bits from bits 2 Q of qh[32 h + l], its scale from
+// sc[8 h + 2 Q + l / 16].
+template <bool F32>
 __global__ __launch_bounds__(256) void dequant_q6k_kernel(const uint8_t* __restrict__ raw, int64_t n_blocks,
                                                           float* __restrict__ out32, uint16_t* __restrict__ out16) {
-  __shared__ __attribute__((aligned(16))) uint8_t span[kQ6Span * 210];
+  __shared__ __attribute__((aligned(16))) uint8_t span[kQ6Span * 210 + 16];
   const int64_t b0 = (int64_t)blockIdx.x * kQ6Span;
   const int nb = (int)min((int64_t)kQ6Span, n_blocks - b0);
   stage_span(raw + b0 * 210, nb * 210, span);
   const int bl = threadIdx.x >> 3, c = threadIdx.x & 7;
   if (bl >= nb) return;
-  const uint8_t* blk = span + bl * 210;
-  const int half = c >> 2, quadrant = c & 3;
-  const float d = h2f((uint16_t)(blk[208] | (blk[209] << 8)));
-  float v[32];
+  const int at = bl * 210;
+  const float d = h2f(*(const uint16_t*)(span + at + 208));
+  const int8_t* sc = (const int8_t*)(span + at + 192);
+  const int64_t o = (b0 + bl) * 256;
 #pragma unroll
-  for (int lane = 0; lane < 32; ++lane) {
-    const uint32_t low = blk[64 * half + lane + 32 * (quadrant & 1)];
-    const uint32_t lowq = quadrant >= 2 ? (low >> 4) : (low & 15u);
-    const uint32_t high = (blk[128 + 32 * half + lane] >> (2 * quadrant)) & 3u;
-    const int scale = (int8_t)blk[192 + 8 * half + (lane >> 4) + 2 * quadrant];
-    v[lane] = (d * (float)scale) * (float)((int)(lowq | (high << 4)) - 32);
-  }
-  const int64_t o = (b0 + bl) * 256 + 128 * half + 32 * quadrant;
-  if (out32) {
+  for (int h = 0; h < 2; ++h) {
+    if constexpr (F32) {
+      const uint32_t qh = lds_word(span, at + 128 + 32 * h + 4 * c);
+      const uint32_t ql[2] = {lds_word(span, at + 64 * h + 4 * c), lds_word(span, at + 64 * h + 32 + 4 * c)};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) *(float4v*)(out32 + o + 4 * i) = float4v{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
-  }
-  if (out16) {
+      for (int Q = 0; Q < 4; ++Q)
+        store_values4(q6k_values4(ql[Q & 1], qh, Q, d * (float)sc[8 * h + 2 * Q + (c >> 2)]),
+                      o + 128 * h + 32 * Q + 4 * c, out32, out16);
+    } else {
+      // values 64 i + 8 c .. +8: quadrant 2 (i % 2) + c / 4, lanes 8 (c % 4) ..
+      const int l = 8 * (c & 3);
+      const uint32_t qh[2] = {lds_word(span, at + 128 + 32 * h + l), lds_word(span, at + 132 + 32 * h + l)};
+      const uint32_t ql[2] = {lds_word(span, at + 64 * h + 8 * c), lds_word(span, at + 64 * h + 8 * c + 4)};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *(half8v*)(out16 + o + 8 * i) = to_half8(v + 8 * i);
+      for (int i = 0; i < 2; ++i) {
+        const int Q = 2 * i + (c >> 2);
+        const float dsc = d * (float)sc[8 * h + 2 * Q + (l >> 4)];
+        const float4v a = q6k_values4(ql[0], qh[0], Q, dsc), b = q6k_values4(ql[1], qh[1], Q, dsc);
+        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        __builtin_nontemporal_store(to_half8(v), (half8v*)(out16 + o + 128 * h + 64 * i + 8 * c));
+      }
+    }
   }
 }
 
-// Q4_0 raw (src/gguf/quantization.ts:40-44): thread t decodes 8 values of
-// block t/4: part p<2 -> low nibbles of bytes 2+8p.., p>=2 -> high nibbles.
+// Q4_0 raw (src/gguf/quantization.ts:40-44): value l < 16 of a block is
+// d * (low nibble of byte 2 + l, less 8), value 16 + l its high nibble.
+__device__ __forceinline__ float4v q40_values4(uint32_t nibbles, float d) {
+  const uint32_t q = opaque(nibbles);
+  return float4v{d * ((float)(q & 0xffu) - 8.0f), d * ((float)((q >> 8) & 0xffu) - 8.0f),
+                 d * ((float)((q >> 16) & 0xffu) - 8.0f), d * ((float)(q >> 24) - 8.0f)};
+}
+
+// A thread's chunks of 4 (float32) or 8 values (f16) lie 256 chunks apart, so
+// every store instruction of a wave is 1 KB of consecutive output.
+template <bool F32>
 __global__ __launch_bounds__(256) void dequant_q40_kernel(const uint8_t* __restrict__ raw, int64_t n_blocks,
                                                           float* __restrict__ out32, uint16_t* __restrict__ out16) {
-  __shared__ __attribute__((aligned(16))) uint8_t span[kQ40Span * 18];
+  __shared__ __attribute__((aligned(16))) uint8_t span[kQ40Span * 18 + 16];
   const int64_t b0 = (int64_t)blockIdx.x * kQ40Span;
   const int nb = (int)min((int64_t)kQ40Span, n_blocks - b0);
   stage_span(raw + b0 * 18, nb * 18, span);
-  const int bl = threadIdx.x >> 2, p = threadIdx.x & 3;
-  if (bl >= nb) return;
-  const uint8_t* blk = span + bl * 18;
-  const float d = h2f((uint16_t)(blk[0] | (blk[1] << 8)));
-  float v[8];
+  constexpr int kChunks = F32 ? 8 : 4;  // per block
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint32_t byte = blk[2 + 8 * (p & 1) + i];
-    const uint32_t q = p >= 2 ? (byte >> 4) : (byte & 15u);
-    v[i] = d * (float)((int)q - 8);
+  for (int it = 0; it < kChunks * kQ40Span / 256; ++it) {
+    const int i = it * 256 + threadIdx.x, bl = i / kChunks, p = i % kChunks;
+    if (bl >= nb) return;
+    const int at = bl * 18, high = p / (kChunks / 2), first = at + 2 + (F32 ? 4 : 8) * (p % (kChunks / 2));
+    const float d = h2f(*(const uint16_t*)(span + at));
+    const int64_t o = (b0 + bl) * 32 + (F32 ? 4 : 8) * p;
+    const float4v a = q40_values4((lds_word(span, first) >> (4 * high)) & 0x0f0f0f0fu, d);
+    if constexpr (F32) {
+      store_values4(a, o, out32, out16);
+    } else {
+      const float4v b = q40_values4((lds_word(span, first + 4) >> (4 * high)) & 0x0f0f0f0fu, d);
+      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      __builtin_nontemporal_store(to_half8(v), (half8v*)(out16 + o));
+    }
   }
-  const int64_t o = (b0 + bl) * 32 + 8 * p;
-  if (out32) {
-    *(float4v*)(out32 + o) = float4v{v[0], v[1], v[2], v[3]};
-    *(float4v*)(out32 + o + 4) = float4v{v[4], v[5], v[6], v[7]};
-  }
-  if (out16) *(half8v*)(out16 + o) = to_half8(v);
 }
 
 hipError_t launch_dequant_raw(int type, const uint8_t* raw, int64_t n_blocks, float* out32, uint16_t* out16,
                               hipStream_t stream) {
   if (n_blocks <= 0) return hipSuccess;
   if (type == kQ4_K) {
-    const int64_t threads = n_blocks * 8;
-    dequant_q4k_kernel<true><<<(unsigned)((threads + 255) / 256), 256, 0, stream>>>(raw, n_blocks, out32, out16);
+    const unsigned grid = (unsigned)((n_blocks * 8 + 255) / 256);
+    if (out32) dequant_q4k_f32_kernel<<<grid, 256, 0, stream>>>(raw, n_blocks, out32, out16);
+    else dequant_q4k_kernel<true><<<grid, 256, 0, stream>>>(raw, n_blocks, out16);
   } else if (type == kQ6_K) {
-    dequant_q6k_kernel<<<(unsigned)((n_blocks + kQ6Span - 1) / kQ6Span), 256, 0, stream>>>(raw, n_blocks, out32, out16);
+    const unsigned grid = (unsigned)((n_blocks + kQ6Span - 1) / kQ6Span);
+    if (out32) dequant_q6k_kernel<true><<<grid, 256, 0, stream>>>(raw, n_blocks, out32, out16);
+    else dequant_q6k_kernel<false><<<grid, 256, 0, stream>>>(raw, n_blocks, nullptr, out16);
   } else if (type == kQ4_0) {
-    dequant_q40_kernel<<<(unsigned)((n_blocks + kQ40Span - 1) / kQ40Span), 256, 0, stream>>>(raw, n_blocks, out32, out16);
+    const unsigned grid = (unsigned)((n_blocks + kQ40Span - 1) / kQ40Span);
+    if (out32) dequant_q40_kernel<true><<<grid, 256, 0, stream>>>(raw, n_blocks, out32, out16);
+    else dequant_q40_kernel<false><<<grid, 256, 0, stream>>>(raw, n_blocks, nullptr, out16);
   } else {
     return hipErrorInvalidValue;
   }
@@ -732,40 +808,39 @@ hipError_t launch_side_expand(const SideExpand& e, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Q6_K split layout -> float32: thread per (block, 32 values).
-__global__ void dequant_q6k_split_kernel(QWeight w, float* __restrict__ out32) {
+// Q6_K split layout -> float32, mapped as dequant_q6k_kernel's float32 form
+// (records are 16-byte aligned here, so the words are read in place).
+__global__ __launch_bounds__(256) void dequant_q6k_split_kernel(QWeight w, float* __restrict__ out32) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nb = (int64_t)w.n * (w.k >> 8);
   const int64_t b = t >> 3;
-  if (b >= nb) return;
-  const int c = (int)(t & 7), half = c >> 2, quadrant = c & 3;
+  if (b >= (int64_t)w.n * (w.k >> 8)) return;
+  const int c = (int)(t & 7);
   const uint8_t* rec = w.blocks + b * 208;
   const float d = h2f(w.d[b]);
-#pragma unroll 4
-  for (int lane = 0; lane < 32; ++lane) {
-    const uint32_t low = rec[64 * half + lane + 32 * (quadrant & 1)];
-    const uint32_t lowq = quadrant >= 2 ? (low >> 4) : (low & 15u);
-    const uint32_t high = (rec[128 + 32 * half + lane] >> (2 * quadrant)) & 3u;
-    const int scale = (int8_t)rec[192 + 8 * half + (lane >> 4) + 2 * quadrant];
-    out32[b * 256 + 128 * half + 32 * quadrant + lane] = (d * (float)scale) * (float)((int)(lowq | (high << 4)) - 32);
+  const u32x4 sc = *(const u32x4*)(rec + 192);
+  const uint32_t scw[4] = {sc.x, sc.y, sc.z, sc.w};
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t qh = *(const uint32_t*)(rec + 128 + 32 * h + 4 * c);
+    const uint32_t ql[2] = {*(const uint32_t*)(rec + 64 * h + 4 * c), *(const uint32_t*)(rec + 64 * h + 32 + 4 * c)};
+#pragma unroll
+    for (int Q = 0; Q < 4; ++Q) {
+      const int si = 8 * h + 2 * Q + (c >> 2);
+      const float dsc = d * (float)(int8_t)((scw[2 * h + (Q >> 1)] >> (8 * (si & 3))) & 0xffu);
+      store_values4(q6k_values4(ql[Q & 1], qh, Q, dsc), b * 256 + 128 * h + 32 * Q + 4 * c, out32, nullptr);
+    }
   }
 }
 
-// Q4_0 split layout: thread per 32-value block.
-__global__ void dequant_q40_split_kernel(QWeight w, int64_t n_blocks, float* __restrict__ out32) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Q4_0 split layout -> float32: thread per 4 values (8 per 32-value block).
+__global__ __launch_bounds__(256) void dequant_q40_split_kernel(QWeight w, int64_t n_blocks,
+                                                                float* __restrict__ out32) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t b = t >> 3;
   if (b >= n_blocks) return;
-  const u32x4 q = *(const u32x4*)(w.blocks + b * 16);
-  const float d = h2f(w.d[b]);
-  const uint32_t words[4] = {q.x, q.y, q.z, q.w};
-  float v[32];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    bytes4_fma(words[i] & 0x0f0f0f0fu, d, -8.0f * d, v + 4 * i);
-    bytes4_fma((words[i] >> 4) & 0x0f0f0f0fu, d, -8.0f * d, v + 16 + 4 * i);
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) *(float4v*)(out32 + b * 32 + 4 * i) = float4v{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+  const int p = (int)(t & 7);
+  const uint32_t q = *(const uint32_t*)(w.blocks + b * 16 + 4 * (p & 3));
+  store_values4(q40_values4((q >> (4 * (p >> 2))) & 0x0f0f0f0fu, h2f(w.d[b])), b * 32 + 4 * p, out32, nullptr);
 }
 
 hipError_t launch_dequant_weight(const QWeight& w, float* out32, hipStream_t stream) {
@@ -773,7 +848,7 @@ hipError_t launch_dequant_weight(const QWeight& w, float* out32, hipStream_t str
   if (w.type == kQ4_K) return launch_dequant_raw(kQ4_K, w.blocks, nb, out32, nullptr, stream);
   if (w.type == kQ4_0) {
     const int64_t n40 = (int64_t)w.n * (w.k / 32);
-    dequant_q40_split_kernel<<<(unsigned)((n40 + 255) / 256), 256, 0, stream>>>(w, n40, out32);
+    dequant_q40_split_kernel<<<(unsigned)((n40 * 8 + 255) / 256), 256, 0, stream>>>(w, n40, out32);
     return hipGetLastError();
   }
   if (w.type != kQ6_K) return hipErrorInvalidValue;
