@@ -310,7 +310,7 @@ struct nemo_plan {
   int batch = 0, sequence = 0, merged = 0;
   hipStream_t stream = nullptr;
   std::mutex mu;
-  DevPtr ids, x_full, norm_full, x_red, norm_red, qkv, attn, delta, ffn, out, rope, partials, wexp;
+  DevPtr ids, x_full, norm_full, x_red, norm_red, qkv, attn, delta, ffn, out, rope, partials, wexp, pool;
   size_t wexp_halves = 0;
   // f16 expansions of a layer's gate/up and down weights, written by the QKV
   // and O GEMM launches on the CUs their tiles leave idle (see
@@ -854,6 +854,7 @@ nemo_status nemo_plan_create(nemo_model* model, int32_t batch, int32_t sequence,
     if (dn) p->wexp_dn = dev_alloc(dn * 2, "f16 down expansion");
     p->wexp_gu_halves = gu;
     p->wexp_dn_halves = dn;
+    p->pool = dev_alloc((size_t)batch * pool_pieces(p->merged) * H * 4, "pooling sums");
     p->out = dev_alloc((size_t)batch * H * 4, "embeddings");
     const std::vector<float> table = rope_table(sequence, d.head_dim, d.rope_theta);
     p->rope = dev_alloc(table.size() * 4, "RoPE sin/cos table");
@@ -979,9 +980,9 @@ static void enqueue_graph(nemo_plan* p, const uint32_t* d_ids, const Ragged& src
   const float* rope = (const float*)p->rope.get();
 
   mark(0, true);
-  hip_check(launch_embed(d_ids, p->sequence, src, m->embedding_type, m->embedding, H, d.vocab, x_full, s), "embedding");
-  hip_check(launch_rmsnorm(x_full, nullptr, m->layers[0].attn_norm, norm_full, src.start[src.count], H, d.rms_epsilon, s),
-            "rmsnorm");
+  hip_check(launch_embed_norm(d_ids, p->sequence, src, m->embedding_type, m->embedding, H, d.vocab, x_full,
+                              m->layers[0].attn_norm, norm_full, d.rms_epsilon, s),
+            "embedding");
   mark(0, false);
   // Whether layer l's QKV and O weights are expanded together into wexp (QKV,
   // then O), and the layer whose expansion the previous down launch did.
@@ -995,8 +996,7 @@ static void enqueue_graph(nemo_plan* p, const uint32_t* d_ids, const Ragged& src
   for (int l = 0; l < d.layers; ++l) {
     if (l == d.merge_after_layer) {
       mark(1, true);
-      hip_check(launch_merge(x_full, src, dst, H, x_red, s), "token merge");
-      hip_check(launch_merge(norm_full, src, dst, H, norm_red, s), "token merge");
+      hip_check(launch_merge(norm_full, x_full, src, dst, H, norm_red, x_red, s), "token merge");
       mark(1, false);
     }
     const bool full = l < d.merge_after_layer;
@@ -1136,11 +1136,11 @@ static void enqueue_graph(nemo_plan* p, const uint32_t* d_ids, const Ragged& src
   }
   if (d.merge_after_layer == d.layers) {  // merge after the last layer (models shorter than the reference)
     mark(1, true);
-    hip_check(launch_merge(norm_full, src, dst, H, norm_red, s), "token merge");
+    hip_check(launch_merge(norm_full, nullptr, src, dst, H, norm_red, nullptr, s), "token merge");
     mark(1, false);
   }
   mark(10, true);
-  hip_check(launch_mean_pool(norm_red, dst, H, d_out, s), "mean pool");
+  hip_check(launch_mean_pool(norm_red, dst, H, (float*)p->pool.get(), d_out, s), "mean pool");
   mark(10, false);
 }
 

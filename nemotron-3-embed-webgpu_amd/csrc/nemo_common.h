@@ -27,21 +27,17 @@ struct Ragged {
   int start[kMaxBatch + 1];
 };
 
-// Per-request work-tile prefix for kernels that tile each request separately
-// (attention query tiles): request b owns tiles [tile[b], tile[b + 1]).
-struct RaggedTiles {
-  int count;
-  int tile[kMaxBatch + 1];
-};
-
 __device__ __forceinline__ float h2f(uint16_t bits) { return (float)__builtin_bit_cast(half_t, bits); }
 __device__ __forceinline__ uint16_t f2h(float v) { return __builtin_bit_cast(uint16_t, (half_t)v); }
 
-// Request index owning packed row t (t < r.start[r.count]).
+// Request index owning packed row t (t < r.start[r.count], the same for the
+// whole wave, every lane active): lane l compares the end of request l, one
+// load instead of a chain of up to 64.
+static_assert(kMaxBatch <= 64, "one lane per request");
 __device__ __forceinline__ int ragged_find(const Ragged& r, int t) {
-  int b = 0;
-  while (b + 1 < r.count && t >= r.start[b + 1]) ++b;
-  return b;
+  const int l = (int)(threadIdx.x & 63);
+  const bool past = l + 1 < r.count && t >= r.start[l + 1];
+  return (int)__popcll(__builtin_amdgcn_ballot_w64(past));
 }
 
 // s_waitcnt immediate waiting for at most `n` outstanding vector memory

@@ -9,13 +9,15 @@
 
 namespace nemo {
 
-// x[t, :] = table row ids[b * padded_seq + p] for packed row t = (b, p).
-// table_type kF16 ([vocab, hidden] f16) or kQ6_K (raw GGUF rows).
-hipError_t launch_embed(const uint32_t* ids, int padded_seq, const Ragged& rows, int table_type, const void* table,
-                        int hidden, int vocab, uint16_t* x, hipStream_t stream);
+// x[t, :] = table row ids[b * padded_seq + p] for packed row t = (b, p), and
+// normalized[t, :] its RMSNorm with weights w. table_type kF16 ([vocab, hidden]
+// f16) or kQ6_K (raw GGUF rows).
+hipError_t launch_embed_norm(const uint32_t* ids, int padded_seq, const Ragged& rows, int table_type,
+                             const void* table, int hidden, int vocab, uint16_t* x, const float* w,
+                             uint16_t* normalized, float eps, hipStream_t stream);
 
-// normalized = f16(f32(x) * rsqrt(mean(v^2) + eps) * w); with delta != null,
-// v = f32(x) + f32(delta) is first stored into x (f16).
+// v = f32(x) + f32(delta) is stored into x (f16), and normalized =
+// f16(v * rsqrt(mean(v^2) + eps) * w) of the stored v.
 hipError_t launch_rmsnorm(uint16_t* x, const uint16_t* delta, const float* w, uint16_t* normalized, int rows,
                           int hidden, float eps, hipStream_t stream);
 
@@ -58,11 +60,15 @@ constexpr int attn_round_keys(int head_dim) { return 16384 / head_dim; }
 // out[t, :F] = f16(silu(g) * u), g = gu[t, :F], u = gu[t, F:2F].
 hipError_t launch_swiglu(const uint16_t* gu, int rows, int f, uint16_t* out, hipStream_t stream);
 
-// Adjacent-state merge of every request from `src` rows to `dst` rows.
-hipError_t launch_merge(const uint16_t* in, const Ragged& src, const Ragged& dst, int hidden, uint16_t* out,
-                        hipStream_t stream);
+// Adjacent-state merge of every request from `src` rows to `dst` rows: the
+// normalized stream and, unless `x` is null, the residual stream.
+hipError_t launch_merge(const uint16_t* norm, const uint16_t* x, const Ragged& src, const Ragged& dst, int hidden,
+                        uint16_t* norm_out, uint16_t* x_out, hipStream_t stream);
 
 // Mean over each request's rows, then L2 normalise; out float [count, hidden].
-hipError_t launch_mean_pool(const uint16_t* norm, const Ragged& rows, int hidden, float* out, hipStream_t stream);
+// `sums`: room for hidden floats per piece, pool_pieces(rows) of each request.
+int pool_pieces(int rows);
+hipError_t launch_mean_pool(const uint16_t* norm, const Ragged& rows, int hidden, float* sums, float* out,
+                            hipStream_t stream);
 
 }  // namespace nemo
