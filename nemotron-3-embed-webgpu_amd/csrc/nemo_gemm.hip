@@ -111,49 +111,76 @@ __device__ __forceinline__ void gemm_epilogue(const float16v (&acc)[MI][4], int 
   }
 }
 
-// The same epilogue for a wave owning MI16 x 8 blocks of 16 x 16 starting at
-// (rbase0, cbase): lane l, register r of block (i, j) is row rbase0 + 16i +
-// 4(l/16) + r, column cbase + 16j + l%16. For kEpiSwiGLU blocks j < 4 are the
-// gate features cbase/2 + 16j + l%16 and blocks j + 4 their up rows.
-template <int EPI, int MI16>
-__device__ __forceinline__ void gemm_epilogue16(const float4v (&acc)[MI16][8], int rbase0, int cbase, int lane, int M,
-                                                int N, void* out, int ldo, int split) {
-  const int rbase = rbase0 + 4 * (lane >> 4);
-  if constexpr (EPI == kEpiSwiGLU) {
-    uint16_t* y = (uint16_t*)out;
+// Epilogue of gemm_f16_kernel, whose MFMAs take the W fragment as their first
+// operand: a lane's accumulators are then features of one token, and with W's
+// LDS rows in f16_w_row's order they are runs of 8 consecutive features, stored
+// with one 16-byte instruction (two for fp32). K16: token 16i + l%16, features
+// 32J + 8(l/16) .. +8 from blocks 2J and 2J + 1; else token 32i + l%32,
+// features 32J + 16c + 8(l/32) .. +8 from registers 8c .. of block J. Rows,
+// columns or pointers that 16-byte stores do not fit go value by value. (With
+// X first, a lane held one column of several tokens and stored 2 bytes at a
+// time, 8 times the store instructions: about 8 us of each round of 256 x 256
+// tiles lay outside the K loop. 500-token request, four layers: 577 -> 554 us,
+// 8 x 1500 tokens 5052 -> 4957, 16 x 150 tokens, 16 layers, 4466 -> 4399.)
+template <bool K16>
+__device__ __forceinline__ int f16_w_row(int p) {
+  const int low = p & 3, b4 = (p >> 4) & 1, b3 = (p >> 3) & 1, b2 = (p >> 2) & 1;
+  return (p & ~31) | (K16 ? 16 * b3 + 8 * b2 + 4 * b4 : 16 * b4 + 8 * b2 + 4 * b3) | low;
+}
+
+template <int EPI, bool K16, int AI, typename Acc, int AJ>
+__device__ __forceinline__ void f16_epilogue(const Acc (&acc)[AI][AJ], int rbase, int cbase, int lane, int M, int N,
+                                             void* out, int ldo, int split) {
+  constexpr bool F32 = EPI == kEpiPartial;
+  constexpr int SPAN = K16 ? 16 : 32, C = K16 ? 1 : 2;  // tokens per block, runs of 8 per lane and 32 features
+  // (SwiGLU goes to the plan's own buffer, whose rows are whole lines.)
+  const bool vec = EPI == kEpiSwiGLU || ((((uintptr_t)out | (uintptr_t)ldo * (F32 ? 4 : 2)) & 15) == 0 && N % 8 == 0);
+  auto value = [&](int i, int J, int c, int e) {
+    if constexpr (K16) return acc[i][2 * J + (e >> 2)][e & 3];
+    else return acc[i][J][8 * c + e];
+  };
 #pragma unroll
-    for (int i = 0; i < MI16; ++i)
+  for (int i = 0; i < AI; ++i) {
+    const int row = rbase + SPAN * i + lane % SPAN;
+    if (row >= M) continue;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int col = (cbase >> 1) + j * 16 + (lane & 15);
+    for (int J = 0; J < (EPI == kEpiSwiGLU ? 2 : 4); ++J)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = rbase + i * 16 + r;
-          if (row < M) {
-            const float g = (float)(half_t)acc[i][j][r];
-            const float u = (float)(half_t)acc[i][j + 4][r];
-            y[(size_t)row * ldo + col] = f2h(g / (1.0f + expf(-g)) * u);
+      for (int c = 0; c < C; ++c) {
+        const int at = 32 * J + 16 * c + 8 * (lane / SPAN);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = value(i, J, c, e);
+        if constexpr (EPI == kEpiSwiGLU) {
+          // Features 0-63 of the wave's 128 are gate rows, 64-127 their up
+          // rows (N % BN == 0). SwiGLU as src/webgpu/ops.ts:85-87 on the
+          // f16-rounded gate/up values.
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float g = (float)(half_t)v[e], u = (float)(half_t)value(i, J + 2, c, e);
+            v[e] = g / (1.0f + expf(-g)) * u;
           }
         }
-      }
-  } else {
+        const int col = (EPI == kEpiSwiGLU ? cbase >> 1 : cbase) + at;
+        const int cols = EPI == kEpiSwiGLU ? N >> 1 : N;
+        if (col >= cols) continue;
+        const size_t o = ((size_t)(EPI == kEpiPartial || EPI == kEpiPartial16 ? split * (size_t)M : 0) + row) * ldo + col;
+        if (vec) {
+          if constexpr (F32) {
+            *(float4v*)((float*)out + o) = float4v{v[0], v[1], v[2], v[3]};
+            *(float4v*)((float*)out + o + 4) = float4v{v[4], v[5], v[6], v[7]};
+          } else {
+            *(half8v*)((uint16_t*)out + o) = to_half8(v);
+          }
+        } else {
 #pragma unroll
-    for (int i = 0; i < MI16; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int col = cbase + j * 16 + (lane & 15);
-        if (col >= N) continue;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = rbase + i * 16 + r;
-          if (row >= M) continue;
-          if constexpr (EPI == kEpiStore)
-            ((uint16_t*)out)[(size_t)row * ldo + col] = f2h(acc[i][j][r]);
-          else if constexpr (EPI == kEpiPartial16)
-            ((uint16_t*)out)[((size_t)split * M + row) * ldo + col] = f2h(acc[i][j][r]);
-          else
-            ((float*)out)[((size_t)split * M + row) * ldo + col] = acc[i][j][r];
+          for (int e = 0; e < 8; ++e)
+            if (col + e < cols) {
+              if constexpr (F32) ((float*)out)[o + e] = v[e];
+              else ((uint16_t*)out)[o + e] = f2h(v[e]);
+            }
         }
+        if constexpr (EPI == kEpiSwiGLU) __builtin_amdgcn_sched_barrier(0);  // one run's temporaries at a time
       }
   }
 }
@@ -651,7 +678,7 @@ __global__ __launch_bounds__(WM * BN / 128 * 64) void gemm_f16_kernel(const uint
 #pragma unroll
   for (int i = 0; i < WI; ++i) {
     const int r = 8 * WI * wave + 8 * i + (lane >> 3);
-    woff[i] = (min(n0 + r, N - 1) - n0) * K + 8 * ((lane & 7) ^ xswz(r));
+    woff[i] = (min(n0 + f16_w_row<K16>(r), N - 1) - n0) * K + 8 * ((lane & 7) ^ xswz(r));
   }
   auto copy = [&](int stage, int k0) {
     const uint16_t* xk = xtile + k0;
@@ -705,7 +732,7 @@ __global__ __launch_bounds__(WM * BN / 128 * 64) void gemm_f16_kernel(const uint
           for (int i = 0; i < AI; ++i)
 #pragma unroll
             for (int j = 0; j < JG; ++j)
-              acc[i][JG * jg + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[j], acc[i][JG * jg + j], 0, 0, 0);
+              acc[i][JG * jg + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[j], af[i], acc[i][JG * jg + j], 0, 0, 0);
           if constexpr (JG == 2) __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -726,7 +753,7 @@ __global__ __launch_bounds__(WM * BN / 128 * 64) void gemm_f16_kernel(const uint
         for (int i = 0; i < MI; ++i)
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[j], af[i], acc[i][j], 0, 0, 0);
       }
     }
   };
@@ -734,12 +761,16 @@ __global__ __launch_bounds__(WM * BN / 128 * 64) void gemm_f16_kernel(const uint
   // The copies of step s+2 are issued right after the barrier that frees
   // their stage and have the whole of step s+1 to land. Loads complete in
   // order: vmcnt(XI + WI) leaves the newer stage's copies in flight.
-  auto kat = [&](int s) { return kbeg + min(s, nsteps - 1) * kBK; };
-  copy(0, kat(0));
-  copy(1, kat(1));
+  copy(0, kbeg);
+  copy(1, kbeg + kBK);
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(XI + WI));
   __syncthreads();
-  for (int s = 0; s < nsteps; s += 2) {
+  // The last two steps copy nothing. The 384 x 256 tile, which has no register
+  // left for them outside its loop, copies its last stage again instead.
+  constexpr bool kPeel = !(WM == 4 && MI == 3);
+  const int last = kPeel ? nsteps - 2 : nsteps;
+  auto kat = [&](int s) { return kbeg + (kPeel ? s : min(s, nsteps - 1)) * kBK; };
+  for (int s = 0; s < last; s += 2) {
     mfma_step(0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -749,11 +780,13 @@ __global__ __launch_bounds__(WM * BN / 128 * 64) void gemm_f16_kernel(const uint
     __syncthreads();
     copy(1, kat(s + 3));
   }
+  if constexpr (kPeel) mfma_step(0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if constexpr (K16)
-    gemm_epilogue16<EPI, AI>(acc, m0 + wm * 32 * MI, n0 + wn * 128, lane, M, N, out, ldo, bz);
-  else
-    gemm_epilogue<EPI, MI>(acc, m0 + wm * 32 * MI, n0 + wn * 128, lane, M, N, out, ldo, bz);
+  if constexpr (kPeel) {
+    __syncthreads();
+    mfma_step(1);
+  }
+  f16_epilogue<EPI, K16, AI>(acc, m0 + wm * 32 * MI, n0 + wn * 128, lane, M, N, out, ldo, bz);
 }
 
 int gemm_splits(const QWeight& w, int m) {
@@ -1069,7 +1102,7 @@ static hipError_t launch_two_pass(const uint16_t* x, int ldx, const QWeight& w, 
                                   void* out, int ldo, uint16_t* wexp, hipStream_t stream, int tile,
                                   bool expanded = false, const SideExpand* side = nullptr) {
   const int bm = f16_bm(tile), bn = f16_bn(tile);
-  if (epilogue == kEpiSwiGLU && w.n % bn) return hipErrorInvalidValue;
+  if (epilogue == kEpiSwiGLU && (w.n % bn || ldo % 8 || ((uintptr_t)out & 15))) return hipErrorInvalidValue;
   // gemm_f16_kernel addresses a tile's rows by 32-bit element offsets
   if ((int64_t)bm * ldx > INT32_MAX || (int64_t)bn * w.k > INT32_MAX) return hipErrorInvalidValue;
   const int64_t threads = (int64_t)w.n * (w.k / 32);
