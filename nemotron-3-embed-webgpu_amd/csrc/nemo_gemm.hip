@@ -85,7 +85,7 @@ __device__ __forceinline__ void gemm_epilogue(const float16v (&acc)[MI][4], int 
           if (row < M) {
             const float g = (float)(half_t)acc[i][j][r];
             const float u = (float)(half_t)acc[i][j + 2][r];
-            y[(size_t)row * ldo + col] = f2h(g / (1.0f + expf(-g)) * u);
+            y[(size_t)row * ldo + col] = f2h(swiglu(g, u));
           }
         }
       }
@@ -158,7 +158,7 @@ __device__ __forceinline__ void f16_epilogue(const Acc (&acc)[AI][AJ], int rbase
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             const float g = (float)(half_t)v[e], u = (float)(half_t)value(i, J + 2, c, e);
-            v[e] = g / (1.0f + expf(-g)) * u;
+            v[e] = swiglu(g, u);
           }
         }
         const int col = (EPI == kEpiSwiGLU ? cbase >> 1 : cbase) + at;
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(const uint16_t* x, int ld
       if (row < M) {
         const float g = (float)(half_t)acc[0][r];
         const float u = (float)(half_t)acc[1][r];
-        y[(size_t)row * ldo + col] = f2h(g / (1.0f + expf(-g)) * u);
+        y[(size_t)row * ldo + col] = f2h(swiglu(g, u));
       }
     }
   } else {
