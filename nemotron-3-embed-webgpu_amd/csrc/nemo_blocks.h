@@ -73,7 +73,6 @@ __device__ __forceinline__ void nibbles4_fma(uint32_t w, float scale, float bias
   out[3] = fmaf(s9, b.y, bias);
 }
 
-// Round-to-nearest-even f32 -> f16 of eight values (v_cvt_pk_f16_f32 pairs).
 // SwiGLU of f16-rounded gate and up values (src/webgpu/ops.ts:85-87) in fp32:
 // g / (1 + e^-g) * u with the hardware exponential and reciprocal (about 1 ulp
 // each; expf and the IEEE division are three times the instructions, and a
@@ -84,6 +83,7 @@ __device__ __forceinline__ float swiglu(float g, float u) {
   return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * g)) * u;
 }
 
+// Round-to-nearest-even f32 -> f16 of eight values (v_cvt_pk_f16_f32 pairs).
 __device__ __forceinline__ half8v to_half8(const float* v) {
   const float8v f = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
   return __builtin_convertvector(f, half8v);

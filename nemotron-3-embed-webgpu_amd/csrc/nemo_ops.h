@@ -42,7 +42,7 @@ hipError_t launch_rope(const uint16_t* qkv, int qkv_stride, const Ragged& rows, 
 // stages the keys and values itself; with `ks` and `vts` (each room for
 // kv_heads * keys_cap * head_dim halves, keys_cap >= attention_prep_keys) a
 // first pass writes the rotated attended keys and the transposed values
-// once, for long requests.
+// once, for long requests. keys_cap is a multiple of 32.
 hipError_t launch_attention(const uint16_t* qkv, int qkv_stride, const float* rope_table, const Ragged& rows,
                             int q_heads, int kv_heads, int head_dim, int stride_threshold, int key_stride, uint16_t* out,
                             hipStream_t stream, uint16_t* ks = nullptr, uint16_t* vts = nullptr, int keys_cap = 0);

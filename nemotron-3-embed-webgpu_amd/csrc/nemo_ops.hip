@@ -333,13 +333,29 @@ __device__ __forceinline__ int attn_keys(int n, int stride_threshold, int key_st
   return (n + s - 1) / s;
 }
 
+constexpr int kAttnLongWaves = 4;
+// Workgroups of a request and KV head: 4 (32-query tile, head) pairs each.
+__host__ __device__ inline int attn_long_workgroups(int n, int group) {
+  return (group * ((n + kAttnQ - 1) / kAttnQ) + kAttnLongWaves - 1) / kAttnLongWaves;
+}
+typedef __attribute__((address_space(3))) void attn_lds_void;
+
 // Long requests: one pass per layer writes each request's attended keys,
-// rotated, as K_s [kv head][key][hd] and its values transposed as
-// V^T_s [kv head][hd][key] (keys of request b from 32 * (sum over earlier
-// requests of ceil(keys / 32)), zero past the last key). The attention's
-// query tiles (157 of them at 5000 tokens) then stage both with 16-byte
-// loads and stores instead of rotating every key again and transposing V
-// with 2-byte LDS stores. Workgroup = 32 keys of one kv head.
+// rotated, and its values transposed, in blocks of 32 keys (request b's from
+// block sum over earlier requests of ceil(keys / 32), zero past its last key),
+// each the LDS image that attention_long_kernel copies as it is:
+//   K_s  [kv head][block][key][16-byte chunk c at c ^ attn_kswz(key)]
+//   V^T_s [kv head][block][d][4 chunks of 8 keys, chunk q at q ^ attn_vswz(d)],
+// chunk q = 2 c2 + hl holding the keys 16 c2 + 8 (e / 4) + 4 hl + e % 4, e =
+// 0..7, that lane half hl's score registers 8 c2 + e hold. The swizzles spread
+// the rows that one fragment read touches over distinct banks. Workgroup = 32
+// keys of one kv head.
+template <int HD>
+__device__ __forceinline__ int attn_kswz(int key) {
+  return HD == 128 ? key & 15 : (key & 7) ^ ((key >> 3) & 1);
+}
+__device__ __forceinline__ int attn_vswz(int d) { return (((d >> 1) ^ (d >> 3)) & 1) | (((d >> 2) & 1) << 1); }
+
 template <int HD>
 __global__ __launch_bounds__(256) void attention_prep_kernel(const uint16_t* __restrict__ qkv, int qkv_stride,
                                                              const float* __restrict__ table, Ragged rows,
@@ -347,7 +363,8 @@ __global__ __launch_bounds__(256) void attention_prep_kernel(const uint16_t* __r
                                                              int key_stride_long, int keys_cap,
                                                              uint16_t* __restrict__ ks, uint16_t* __restrict__ vts) {
   __shared__ __attribute__((aligned(16))) half_t sv[kAttnKeys * (HD + 8)];
-  int b = 0, blk = blockIdx.x;
+  const int kvh = blockIdx.x % kv_heads, block = blockIdx.x / kv_heads;
+  int b = 0, blk = block;
   for (; b < rows.count; ++b) {
     const int blocks = (attn_keys(rows.start[b + 1] - rows.start[b], stride_threshold, key_stride_long) + 31) / 32;
     if (blk < blocks) break;
@@ -357,7 +374,7 @@ __global__ __launch_bounds__(256) void attention_prep_kernel(const uint16_t* __r
   const int row0 = rows.start[b], n = rows.start[b + 1] - row0;
   const int key_stride = n > stride_threshold ? key_stride_long : 1;
   const int n_keys = (n + key_stride - 1) / key_stride;
-  const int kvh = blockIdx.y, g0 = kAttnKeys * blockIdx.x;  // first key of this block in the buffers
+  const size_t image = ((size_t)kvh * keys_cap + kAttnKeys * block) * HD;  // this block in either buffer
   const uint16_t* kbase = qkv + (q_heads + kvh) * HD;
   const uint16_t* vbase = qkv + (q_heads + kv_heads + kvh) * HD;
   for (int i = threadIdx.x; i < kAttnKeys * HD / 8; i += blockDim.x) {
@@ -369,80 +386,39 @@ __global__ __launch_bounds__(256) void attention_prep_kernel(const uint16_t* __r
       kv = rope8(*(const half8v*)(kbase + trow + c), table + (size_t)kpos * HD + c);
       vv = *(const half8v*)(vbase + trow + c);
     }
-    *(half8v*)(ks + ((size_t)kvh * keys_cap + g0 + j) * HD + c) = kv;
+    *(half8v*)(ks + image + j * HD + 8 * ((c >> 3) ^ attn_kswz<HD>(j))) = kv;
     *(half8v*)&sv[j * (HD + 8) + c] = vv;
   }
   __syncthreads();
   for (int i = threadIdx.x; i < HD * kAttnKeys / 8; i += blockDim.x) {
-    const int d = i / (kAttnKeys / 8), k0 = (i % (kAttnKeys / 8)) * 8;
+    const int d = i / (kAttnKeys / 8), q = i % (kAttnKeys / 8);
     half8v col;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) col[r] = sv[(k0 + r) * (HD + 8) + d];
-    *(half8v*)(vts + ((size_t)kvh * HD + d) * keys_cap + g0 + k0) = col;
+    for (int e = 0; e < 8; ++e) col[e] = sv[(16 * (q >> 1) + 8 * (e >> 2) + 4 * (q & 1) + (e & 3)) * (HD + 8) + d];
+    *(half8v*)(vts + image + d * kAttnKeys + 8 * (q ^ attn_vswz(d))) = col;
   }
 }
 
-// Fewest threads per block that the prepared path's staging supports.
-constexpr int attn_prep_min_threads(int hd) { return hd == 128 ? 128 : 64; }
-
-template <int HD, bool PREP>
-__global__ __launch_bounds__(512) void attention_kernel(const uint16_t* __restrict__ qkv, int qkv_stride,
-                                                        const float* __restrict__ table, Ragged rows, int q_heads,
-                                                        int kv_heads, int stride_threshold, int key_stride_long,
-                                                        const uint16_t* __restrict__ ks,
-                                                        const uint16_t* __restrict__ vts, int keys_cap, int sb_keys,
-                                                        uint16_t* __restrict__ out) {
-  constexpr int KP = HD + 8;  // padded K row (halves)
-  constexpr int DC = HD / 16; // 16-wide d chunks of the score MFMAs
-  constexpr int DB = HD / 32; // 32-wide d blocks of the output
-  // sb_keys (a multiple of 32) keys are staged per round: sK [sb_keys][KP],
-  // sVt [HD][VP].
-  extern __shared__ __attribute__((aligned(16))) uint8_t attn_lds[];
-  const int VP = sb_keys + 8;
-  half_t* sK = (half_t*)attn_lds;
-  half_t* sVt = sK + sb_keys * KP;
-  int b = 0, tile = blockIdx.x, koff = 0;  // koff: the request's first key in K_s / V^T_s
-  for (; b < rows.count; ++b) {
-    const int n = rows.start[b + 1] - rows.start[b];
-    const int tiles = (n + kAttnQ - 1) / kAttnQ;
-    if (tile < tiles) break;
-    tile -= tiles;
-    koff += kAttnKeys * ((attn_keys(n, stride_threshold, key_stride_long) + kAttnKeys - 1) / kAttnKeys);
-  }
-  if (b >= rows.count) return;
-  const int row0 = rows.start[b];
-  const int n = rows.start[b + 1] - row0;
-  const int kvh = blockIdx.y;
-  const int group = q_heads / kv_heads;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hl = lane >> 5;
-  const int h = kvh * group + wave;
-  const int qi = tile * kAttnQ + (lane & 31);
-  const int key_stride = n > stride_threshold ? key_stride_long : 1;
-  const int n_keys = (n + key_stride - 1) / key_stride;
-  const float temperature = qi >= 16384 ? logf(floorf((float)qi / 16384.0f) + 1.0f) * 0.1f + 1.0f : 1.0f;
-  const float scale2 = (1.0f / sqrtf((float)HD)) * temperature * 1.4426950408889634f;
-
-  half8v qf[DC];
-  {
-    const int qpos = min(qi, n - 1);
-    const uint16_t* qp = qkv + (size_t)(row0 + qpos) * qkv_stride + h * HD + 8 * hl;
-    const float* cs = table + (size_t)qpos * HD + 8 * hl;
-#pragma unroll
-    for (int c = 0; c < DC; ++c) qf[c] = rope8(*(const half8v*)(qp + 16 * c), cs + 16 * c);
-  }
-  const uint16_t* kbase = qkv + (q_heads + kvh) * HD;
-  const uint16_t* vbase = qkv + (q_heads + kv_heads + kvh) * HD;
+// A wave's 32 queries of one head: query l%32 in lane l, whose half hl = l/32
+// holds d 32db + 8j + 4hl + 0..3 in registers 4j.. of o[db], and the sum of its
+// own keys' probabilities. m: the query's reference maximum (log2 units,
+// scaled).
+template <int HD>
+struct AttnRows {
+  static constexpr int DB = HD / 32;  // 32-wide d blocks of the output
   float16v o[DB];
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
-  // m: the query's reference maximum (log2 units, scaled); lsum: the sum of
-  // this half's probabilities (the two halves' are added at the end).
   float m = -INFINITY, lsum = 0.f;
 
-  // One block of kAttnKeys staged keys from key kb of cK [keys][KP] and
-  // cV [HD][vp]; keys at or past `staged` are masked.
+  __device__ __forceinline__ AttnRows() {
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
+  }
+
+  // The probabilities of one block of 32 keys, as the B operands of its two
+  // 16-key chunks: s register r is the score of key 8(r/4) + 4hl + r%4, of
+  // which the first `valid` exist.
   //
   // Probabilities are taken against a reference maximum m that is raised
   // only when a query's block maximum exceeds it by more than 2^8 (a wave
@@ -451,21 +427,12 @@ __global__ __launch_bounds__(512) void attention_kernel(const uint16_t* __restri
   // exchange, no rescale of the accumulators and no 2^(m - m') of its own.
   // The result is the softmax all the same: numerator and denominator share
   // the reference.
-  auto block = [&](const half_t* cK, const half_t* cV, int vp, int kb, int staged) {
-    // S^T block: lane holds query l%32, key kb + 8(r/4) + 4hl + r%4.
-    float16v s;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = 0.f;
-#pragma unroll
-    for (int c = 0; c < DC; ++c) {
-      const half8v a = *(const half8v*)&cK[(kb + (lane & 31)) * KP + 16 * c + 8 * hl];
-      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[c], s, 0, 0, 0);
-    }
-    if (kb + kAttnKeys > staged) {  // the request's last keys: mask past its end
-      asm volatile("");  // keeps this rare path a branch (not computed and selected every block)
+  __device__ __forceinline__ void probabilities(float16v s, float scale2, int valid, int hl, half8v (&pb)[2]) {
+    if (valid < kAttnKeys) {  // the request's last keys: mask past its end
+      asm volatile("");       // keeps this rare path a branch (not computed and selected every block)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        if (kb + 8 * (r >> 2) + 4 * hl + (r & 3) >= staged) s[r] = -INFINITY;
+        if (8 * (r >> 2) + 4 * hl + (r & 3) >= valid) s[r] = -INFINITY;
     }
     float bm = s[0];
 #pragma unroll
@@ -489,126 +456,255 @@ __global__ __launch_bounds__(512) void attention_kernel(const uint16_t* __restri
       p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], scale2, -m));
       lsum += p[r];
     }
+    pb[0] = to_half8(p);
+    pb[1] = to_half8(p + 8);
+  }
+
+  __device__ __forceinline__ void store(uint16_t* __restrict__ op, int hl) {
+    const float inv = 1.0f / lsum;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const half4v hv = {(half_t)(o[db][4 * j] * inv), (half_t)(o[db][4 * j + 1] * inv),
+                           (half_t)(o[db][4 * j + 2] * inv), (half_t)(o[db][4 * j + 3] * inv)};
+        *(half4v*)(op + 32 * db + 8 * j + 4 * hl) = hv;
+      }
+  }
+};
+
+// Query fragments of one head (16-wide d chunks), rotated; and the scores'
+// factor in log2 units.
+template <int HD>
+__device__ __forceinline__ void attn_queries(const uint16_t* __restrict__ qkv, int qkv_stride,
+                                             const float* __restrict__ table, int row0, int qpos, int h, int hl,
+                                             half8v (&qf)[HD / 16]) {
+  const uint16_t* qp = qkv + (size_t)(row0 + qpos) * qkv_stride + h * HD + 8 * hl;
+  const float* cs = table + (size_t)qpos * HD + 8 * hl;
+#pragma unroll
+  for (int c = 0; c < HD / 16; ++c) qf[c] = rope8(*(const half8v*)(qp + 16 * c), cs + 16 * c);
+}
+template <int HD>
+__device__ __forceinline__ float attn_scale2(int qi) {
+  const float temperature = qi >= 16384 ? logf(floorf((float)qi / 16384.0f) + 1.0f) * 0.1f + 1.0f : 1.0f;
+  return (1.0f / sqrtf((float)HD)) * temperature * 1.4426950408889634f;
+}
+
+// Requests of at most one staging round of keys (and any when the key images
+// are not there): keys and values staged from the QKV projection.
+template <int HD>
+__global__ __launch_bounds__(512) void attention_kernel(const uint16_t* __restrict__ qkv, int qkv_stride,
+                                                        const float* __restrict__ table, Ragged rows, int q_heads,
+                                                        int kv_heads, int stride_threshold, int key_stride_long,
+                                                        int sb_keys, uint16_t* __restrict__ out) {
+  constexpr int KP = HD + 8;  // padded K row (halves)
+  constexpr int DC = HD / 16; // 16-wide d chunks of the score MFMAs
+  constexpr int DB = HD / 32; // 32-wide d blocks of the output
+  // sb_keys (a multiple of 32) keys are staged per round: sK [sb_keys][KP],
+  // sVt [HD][VP].
+  extern __shared__ __attribute__((aligned(16))) uint8_t attn_lds[];
+  const int VP = sb_keys + 8;
+  half_t* sK = (half_t*)attn_lds;
+  half_t* sVt = sK + sb_keys * KP;
+  const int kvh = blockIdx.x % kv_heads;  // fastest: a KV head's workgroups share an XCD's L2
+  int b = 0, tile = blockIdx.x / kv_heads;
+  for (; b < rows.count; ++b) {
+    const int tiles = (rows.start[b + 1] - rows.start[b] + kAttnQ - 1) / kAttnQ;
+    if (tile < tiles) break;
+    tile -= tiles;
+  }
+  if (b >= rows.count) return;
+  const int row0 = rows.start[b];
+  const int n = rows.start[b + 1] - row0;
+  const int group = q_heads / kv_heads;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hl = lane >> 5;
+  const int h = kvh * group + wave;
+  const int qi = tile * kAttnQ + (lane & 31);
+  const int key_stride = n > stride_threshold ? key_stride_long : 1;
+  const int n_keys = (n + key_stride - 1) / key_stride;
+  const float scale2 = attn_scale2<HD>(qi);
+  half8v qf[DC];
+  attn_queries<HD>(qkv, qkv_stride, table, row0, min(qi, n - 1), h, hl, qf);
+  const uint16_t* kbase = qkv + (q_heads + kvh) * HD;
+  const uint16_t* vbase = qkv + (q_heads + kv_heads + kvh) * HD;
+  AttnRows<HD> acc;
+
+  // The block of staged keys from kb; keys at or past `staged` are masked.
+  auto block = [&](int kb, int staged) {
+    float16v s = {};
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+      const half8v a = *(const half8v*)&sK[(kb + (lane & 31)) * KP + 16 * c + 8 * hl];
+      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[c], s, 0, 0, 0);
+    }
+    half8v pb[2];
+    acc.probabilities(s, scale2, staged - kb, hl, pb);
     // O^T += V^T P^T over two 16-key chunks: MFMA k slot 8hl + e of chunk c2
     // is key 16c2 + 8(e/4) + 4hl + e%4 = score register 8c2 + e.
 #pragma unroll
-    for (int c2 = 0; c2 < 2; ++c2) {
-      const half8v pb = to_half8(p + 8 * c2);
+    for (int c2 = 0; c2 < 2; ++c2)
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        const half_t* vr = &cV[(32 * db + (lane & 31)) * vp + kb + 16 * c2 + 4 * hl];
+        const half_t* vr = &sVt[(32 * db + (lane & 31)) * VP + kb + 16 * c2 + 4 * hl];
         const half4v v0 = *(const half4v*)vr;
         const half4v v1 = *(const half4v*)(vr + 8);
         const half8v a = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb, o[db], 0, 0, 0);
+        acc.o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[c2], acc.o[db], 0, 0, 0);
+      }
+  };
+  for (int sb = 0; sb < n_keys; sb += sb_keys) {
+    const int staged = min(sb_keys, n_keys - sb);
+    __syncthreads();
+    // 16-byte chunks of the staged keys (rows past `staged` up to the
+    // next multiple of 32 are zero), in batches of 4 per thread with every
+    // load of a batch issued before the first is used.
+    const int chunks = (staged + 31) / 32 * 32 * HD / 8;
+    for (int i0 = threadIdx.x; i0 < chunks; i0 += 4 * blockDim.x) {
+      half8v kr[4], vr[4];
+      float4v ca[4], cb[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = i0 + u * blockDim.x, j = i / (HD / 8), c = (i % (HD / 8)) * 8;
+        kr[u] = half8v{};
+        vr[u] = half8v{};
+        ca[u] = cb[u] = float4v{0.f, 0.f, 0.f, 0.f};
+        if (i < chunks && j < staged) {
+          const int kpos = (sb + j) * key_stride;
+          const size_t trow = (size_t)(row0 + kpos) * qkv_stride;
+          kr[u] = *(const half8v*)(kbase + trow + c);
+          vr[u] = *(const half8v*)(vbase + trow + c);
+          const float* cs = table + (size_t)kpos * HD + c;
+          ca[u] = *(const float4v*)cs;
+          cb[u] = *(const float4v*)(cs + 4);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = i0 + u * blockDim.x, j = i / (HD / 8), c = (i % (HD / 8)) * 8;
+        if (i < chunks) {
+          *(half8v*)&sK[j * KP + c] = rope8(kr[u], ca[u], cb[u]);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) sVt[(c + e) * VP + j] = vr[u][e];
+        }
+      }
+    }
+    __syncthreads();
+    for (int kb = 0; kb < staged; kb += kAttnKeys) block(kb, staged);
+  }
+  acc.lsum += __shfl_xor(acc.lsum, 32, 64);  // the two halves' keys (same references)
+  if (qi < n) acc.store(out + ((size_t)(row0 + qi) * q_heads + h) * HD, hl);
+}
+
+// Longer requests, on the key images of attention_prep_kernel. Workgroup = 4
+// waves = 4 consecutive (32-query tile, head of the group) pairs of one
+// request and KV head; 64 keys per round (two images of 32), copied global ->
+// LDS in two stages, one barrier per round, the copies of round r + 1 in
+// flight under round r. The two blocks' score chains are independent, and one
+// block's exponentials run under the other's MFMAs.
+//
+// Bound by the LDS reads (1 KB per MFMA, as long as the MFMA takes on four
+// SIMDs) and the exponentials together. What it replaced staged 32 keys per
+// barrier through registers for one workgroup of `group` waves (3 at the
+// published heads: 6 waves on a CU, on 2 of its SIMDs 2): 8 x 1500 tokens,
+// 24 heads of 128, 458 -> 277 us a layer; 5000 tokens, 32 heads of 64, every
+// third key, 109 -> 101, 3200 64 -> 53 (same bits). The KV head runs fastest in the grid, so with 8 of
+// them each XCD's L2 holds the images of one.
+template <int HD>
+__global__ __launch_bounds__(256, HD == 128 ? 2 : 4)
+void attention_long_kernel(const uint16_t* __restrict__ qkv, int qkv_stride, const float* __restrict__ table,
+                           Ragged rows, int q_heads, int kv_heads, int stride_threshold, int key_stride_long,
+                           const uint16_t* __restrict__ ks, const uint16_t* __restrict__ vts, int keys_cap,
+                           uint16_t* __restrict__ out) {
+  constexpr int DC = HD / 16, DB = HD / 32;
+  constexpr int IMG = 2 * kAttnKeys * HD;  // bytes of an image of 32 keys
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2][2][2 * IMG];  // [stage][block]: K, then V^T
+  const int group = q_heads / kv_heads;
+  const int kvh = blockIdx.x % kv_heads;
+  int b = 0, wg = blockIdx.x / kv_heads, koff = 0;  // koff: the request's first key in the images
+  for (; b < rows.count; ++b) {
+    const int n = rows.start[b + 1] - rows.start[b];
+    const int wgs = attn_long_workgroups(n, group);
+    if (wg < wgs) break;
+    wg -= wgs;
+    koff += kAttnKeys * ((attn_keys(n, stride_threshold, key_stride_long) + kAttnKeys - 1) / kAttnKeys);
+  }
+  if (b >= rows.count) return;
+  const int row0 = rows.start[b];
+  const int n = rows.start[b + 1] - row0;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), hl = lane >> 5;
+  const int item = kAttnLongWaves * wg + wave;
+  const bool active = item < group * ((n + kAttnQ - 1) / kAttnQ);  // uniform in the wave
+  const int tile = active ? item / group : 0;
+  const int h = kvh * group + item % group;
+  const int qi = tile * kAttnQ + (lane & 31);
+  const int n_keys = attn_keys(n, stride_threshold, key_stride_long);
+  const int blocks = (n_keys + kAttnKeys - 1) / kAttnKeys, rounds = (blocks + 1) >> 1;
+
+  const size_t first = ((size_t)kvh * keys_cap + koff) * HD;
+  auto stage = [&](int r) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (2 * r + u >= blocks) break;
+      const size_t image = first + (size_t)(2 * r + u) * kAttnKeys * HD;
+      uint8_t* dst = lds[r & 1][u];
+#pragma unroll
+      for (int i = 0; i < HD / 64; ++i) {  // 1 KB per instruction
+        const int at = 1024 * (HD / 64 * wave + i);
+        __builtin_amdgcn_global_load_lds((const void*)(ks + image + at / 2 + 8 * lane), (attn_lds_void*)(dst + at), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void*)(vts + image + at / 2 + 8 * lane),
+                                         (attn_lds_void*)(dst + IMG + at), 16, 0, 0);
       }
     }
   };
-  if constexpr (PREP) {
-    // Rounds of kAttnKeys keys from K_s / V^T_s (zero-padded to whole
-    // rounds), double-buffered in LDS: each thread's 16-byte chunks of
-    // round r + 2 are loaded into registers while round r is computed and
-    // stored after it, so one barrier per round remains and a round's loads
-    // have a whole round to land.
-    constexpr int RK = kAttnKeys, VPR = RK + 8;
-    constexpr int KCH = RK * HD / 8, VCH = HD * (RK / 8);  // chunks of a round's K rows and V^T rows
-    constexpr int U = KCH / attn_prep_min_threads(HD);      // slots per thread at the smallest block
-    static_assert(KCH == VCH && KCH % attn_prep_min_threads(HD) == 0, "K and V^T chunks share the slots");
-    constexpr int STAGE = RK * KP + HD * VPR;               // halves per LDS stage
-    const int rounds = (n_keys + RK - 1) / RK;
-    const uint16_t* kp = ks + ((size_t)kvh * keys_cap + koff) * HD;
-    const uint16_t* vp0 = vts + (size_t)kvh * HD * keys_cap + koff;
-    half8v kr[U], vr[U];
-    auto load = [&](int r) {
+  stage(0);
+  const float scale2 = attn_scale2<HD>(qi);
+  half8v qf[DC];
+  attn_queries<HD>(qkv, qkv_stride, table, row0, min(qi, n - 1), h, hl, qf);
+  AttnRows<HD> acc;
+  const int krow = (lane & 31) * HD * 2, ksw = attn_kswz<HD>(lane & 31);
+  const int vrow = IMG + (lane & 31) * kAttnKeys * 2, vsw = attn_vswz(lane & 31);  // rows 32 apart share the swizzle
+  auto score = [&](const uint8_t* img, int c, float16v& s) {
+    const half8v a = *(const half8v*)(img + krow + 16 * ((2 * c + hl) ^ ksw));
+    s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[c], s, 0, 0, 0);
+  };
+  auto values = [&](const uint8_t* img, const half8v (&pb)[2]) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = threadIdx.x + u * blockDim.x;
-        if (i < KCH) {
-          kr[u] = *(const half8v*)(kp + (size_t)r * RK * HD + 8 * i);
-          const int d = i / (RK / 8), k0 = (i % (RK / 8)) * 8;
-          vr[u] = *(const half8v*)(vp0 + (size_t)d * keys_cap + r * RK + k0);
-        }
+    for (int c2 = 0; c2 < 2; ++c2)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        const half8v a = *(const half8v*)(img + vrow + db * 32 * kAttnKeys * 2 + 16 * ((2 * c2 + hl) ^ vsw));
+        acc.o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[c2], acc.o[db], 0, 0, 0);
       }
-    };
-    auto store = [&](int stage) {
-      half_t* dK = sK + stage * STAGE;
-      half_t* dV = dK + RK * KP;
+  };
+  for (int r = 0; r < rounds; ++r) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();  // round r has landed, and every wave has left the other stage
+    if (r + 1 < rounds) stage(r + 1);
+    if (!active) continue;
+    const uint8_t* i0 = lds[r & 1][0];
+    const uint8_t* i1 = lds[r & 1][1];
+    const int valid = n_keys - 2 * kAttnKeys * r;
+    half8v pb[2];
+    float16v s0 = {}, s1 = {};
+    if (valid > kAttnKeys) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = threadIdx.x + u * blockDim.x;
-        if (i < KCH) {
-          *(half8v*)&dK[(i / (HD / 8)) * KP + (i % (HD / 8)) * 8] = kr[u];
-          *(half8v*)&dV[(i / (RK / 8)) * VPR + (i % (RK / 8)) * 8] = vr[u];
-        }
+      for (int c = 0; c < DC; ++c) {
+        score(i0, c, s0);
+        score(i1, c, s1);
       }
-    };
-    load(0);
-    store(0);
-    if (rounds > 1) load(1);
-    __syncthreads();
-    for (int r = 0; r < rounds; ++r) {
-      const half_t* cK = sK + (r & 1) * STAGE;
-      block(cK, cK + RK * KP, VPR, 0, min(RK, n_keys - r * RK));
-      if (r + 1 < rounds) {
-        store((r + 1) & 1);
-        if (r + 2 < rounds) load(r + 2);
-      }
-      __syncthreads();
-    }
-  } else {
-    for (int sb = 0; sb < n_keys; sb += sb_keys) {
-      const int staged = min(sb_keys, n_keys - sb);
-      __syncthreads();
-      // 16-byte chunks of the staged keys (rows past `staged` up to the
-      // next multiple of 32 are zero), in batches of 4 per thread with every
-      // load of a batch issued before the first is used.
-      const int chunks = (staged + 31) / 32 * 32 * HD / 8;
-      for (int i0 = threadIdx.x; i0 < chunks; i0 += 4 * blockDim.x) {
-        half8v kr[4], vr[4];
-        float4v ca[4], cb[4];
+      acc.probabilities(s0, scale2, kAttnKeys, hl, pb);
+      values(i0, pb);
+      acc.probabilities(s1, scale2, valid - kAttnKeys, hl, pb);
+      values(i1, pb);
+    } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int i = i0 + u * blockDim.x, j = i / (HD / 8), c = (i % (HD / 8)) * 8;
-          kr[u] = half8v{};
-          vr[u] = half8v{};
-          ca[u] = cb[u] = float4v{0.f, 0.f, 0.f, 0.f};
-          if (i < chunks && j < staged) {
-            const int kpos = (sb + j) * key_stride;
-            const size_t trow = (size_t)(row0 + kpos) * qkv_stride;
-            kr[u] = *(const half8v*)(kbase + trow + c);
-            vr[u] = *(const half8v*)(vbase + trow + c);
-            const float* cs = table + (size_t)kpos * HD + c;
-            ca[u] = *(const float4v*)cs;
-            cb[u] = *(const float4v*)(cs + 4);
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int i = i0 + u * blockDim.x, j = i / (HD / 8), c = (i % (HD / 8)) * 8;
-          if (i < chunks) {
-            *(half8v*)&sK[j * KP + c] = rope8(kr[u], ca[u], cb[u]);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) sVt[(c + e) * VP + j] = vr[u][e];
-          }
-        }
-      }
-      __syncthreads();
-      for (int kb = 0; kb < staged; kb += kAttnKeys) block(sK, sVt, VP, kb, staged);
+      for (int c = 0; c < DC; ++c) score(i0, c, s0);
+      acc.probabilities(s0, scale2, valid, hl, pb);
+      values(i0, pb);
     }
   }
-  lsum += __shfl_xor(lsum, 32, 64);  // the two halves' keys (same references)
-  if (qi >= n) return;
-  const float inv = 1.0f / lsum;
-  uint16_t* op = out + ((size_t)(row0 + qi) * q_heads + h) * HD;
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      // registers 4j..4j+3 hold d = 32db + 8j + 4hl + 0..3 (contiguous)
-      const half4v hv = {(half_t)(o[db][4 * j] * inv), (half_t)(o[db][4 * j + 1] * inv),
-                         (half_t)(o[db][4 * j + 2] * inv), (half_t)(o[db][4 * j + 3] * inv)};
-      *(half4v*)(op + 32 * db + 8 * j + 4 * hl) = hv;
-    }
+  acc.lsum += __shfl_xor(acc.lsum, 32, 64);  // the two halves' keys (same references)
+  if (active && qi < n) acc.store(out + ((size_t)(row0 + qi) * q_heads + h) * HD, hl);
 }
 
 int attention_prep_keys(const Ragged& rows, int stride_threshold, int key_stride) {
@@ -624,60 +720,51 @@ int attention_prep_keys(const Ragged& rows, int stride_threshold, int key_stride
 hipError_t launch_attention(const uint16_t* qkv, int qkv_stride, const float* rope_table, const Ragged& rows,
                             int q_heads, int kv_heads, int head_dim, int stride_threshold, int key_stride, uint16_t* out,
                             hipStream_t stream, uint16_t* ks, uint16_t* vts, int keys_cap) {
-  int tiles = 0;
-  for (int b = 0; b < rows.count; ++b) tiles += (rows.start[b + 1] - rows.start[b] + kAttnQ - 1) / kAttnQ;
-  if (tiles == 0) return hipSuccess;
-  const int group = q_heads / kv_heads;
+  int tiles = 0, wgs = 0, longest_keys = 0;
+  const int group = kv_heads > 0 ? q_heads / kv_heads : 0;
   if (group < 1 || group > 8 || q_heads % kv_heads) return hipErrorInvalidValue;
   if (head_dim != 64 && head_dim != 128) return hipErrorInvalidValue;
-  // The prepared path's register slots cover a round with 64 threads per
-  // 16 dims of the head (one wave at head_dim 64, two at 128); smaller
-  // blocks stage from the projection instead.
-  const bool prep = ks != nullptr && 64 * group >= attn_prep_min_threads(head_dim);
-  if (prep) {
-    const int keys = attention_prep_keys(rows, stride_threshold, key_stride);
-    if (!vts || keys > keys_cap) return hipErrorInvalidValue;
-    dim3 pgrid(keys / kAttnKeys, kv_heads);
-    if (head_dim == 64)
-      attention_prep_kernel<64><<<pgrid, 256, 0, stream>>>(qkv, qkv_stride, rope_table, rows, q_heads, kv_heads,
-                                                           stride_threshold, key_stride, keys_cap, ks, vts);
-    else
-      attention_prep_kernel<128><<<pgrid, 256, 0, stream>>>(qkv, qkv_stride, rope_table, rows, q_heads, kv_heads,
-                                                            stride_threshold, key_stride, keys_cap, ks, vts);
-  }
-  dim3 grid(tiles, kv_heads);
-  // Keys staged per round: every key of the pass's longest request when
-  // they fit in ~72 KB of LDS and short requests only (one round of loads
-  // and barriers instead of one per 32 keys); 32 for the prepared path, in
-  // two LDS stages.
-  int longest_keys = 0;
   for (int b = 0; b < rows.count; ++b) {
     const int n = rows.start[b + 1] - rows.start[b];
+    tiles += (n + kAttnQ - 1) / kAttnQ;
+    wgs += attn_long_workgroups(n, group);
     const int s = n > stride_threshold ? key_stride : 1;
     longest_keys = std::max(longest_keys, (n + s - 1) / s);
   }
-  const int cap = attn_round_keys(head_dim);
-  const int sb = prep ? kAttnKeys : std::min(cap, (longest_keys + kAttnKeys - 1) / kAttnKeys * kAttnKeys);
-  const int lds = (prep ? 2 : 1) * 2 * (sb * (head_dim + 8) + head_dim * (sb + 8));  // prepared: two stages
-#define NEMO_ATTN(HD, P)                                                                                           \
-  attention_kernel<HD, P><<<grid, 64 * group, lds, stream>>>(qkv, qkv_stride, rope_table, rows, q_heads, kv_heads, \
-                                                             stride_threshold, key_stride, ks, vts, keys_cap, sb, out)
-  auto attr = [&](const void* kernel) {
-    static bool configured[4] = {false, false, false, false};  // one attribute call per instantiation
-    const int slot = (head_dim == 64 ? 0 : 2) + (prep ? 1 : 0);
-    if (!configured[slot]) {
-      (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (cap * (head_dim + 8) + head_dim * (cap + 8)));
-      configured[slot] = true;
-    }
-  };
-  if (head_dim == 64) {
-    if (prep) { attr((const void*)attention_kernel<64, true>); NEMO_ATTN(64, true); }
-    else { attr((const void*)attention_kernel<64, false>); NEMO_ATTN(64, false); }
-  } else {
-    if (prep) { attr((const void*)attention_kernel<128, true>); NEMO_ATTN(128, true); }
-    else { attr((const void*)attention_kernel<128, false>); NEMO_ATTN(128, false); }
+  if (tiles == 0) return hipSuccess;
+  if (ks != nullptr) {
+    const int keys = attention_prep_keys(rows, stride_threshold, key_stride);
+    if (!vts || keys > keys_cap || keys_cap % kAttnKeys) return hipErrorInvalidValue;
+    const unsigned pgrid = (unsigned)kv_heads * (keys / kAttnKeys), grid = (unsigned)kv_heads * wgs;
+    auto launch = [&](auto prep, auto attend) {
+      prep<<<pgrid, 256, 0, stream>>>(qkv, qkv_stride, rope_table, rows, q_heads, kv_heads, stride_threshold,
+                                      key_stride, keys_cap, ks, vts);
+      attend<<<grid, 64 * kAttnLongWaves, 0, stream>>>(qkv, qkv_stride, rope_table, rows, q_heads, kv_heads,
+                                                       stride_threshold, key_stride, ks, vts, keys_cap, out);
+    };
+    if (head_dim == 64) launch(attention_prep_kernel<64>, attention_long_kernel<64>);
+    else launch(attention_prep_kernel<128>, attention_long_kernel<128>);
+    return hipGetLastError();
   }
-#undef NEMO_ATTN
+  const unsigned grid = (unsigned)kv_heads * tiles;
+  // Keys staged per round: every key of the pass's longest request when
+  // they fit in ~72 KB of LDS (one round of loads and barriers instead of one
+  // per 32 keys).
+  const int cap = attn_round_keys(head_dim);
+  const int sb = std::min(cap, (longest_keys + kAttnKeys - 1) / kAttnKeys * kAttnKeys);
+  const int lds = 2 * (sb * (head_dim + 8) + head_dim * (sb + 8));
+  auto launch = [&](auto kernel) {
+    static bool configured = false;  // one attribute call per instantiation
+    if (!configured) {
+      (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                2 * (cap * (head_dim + 8) + head_dim * (cap + 8)));
+      configured = true;
+    }
+    kernel<<<grid, 64 * group, lds, stream>>>(qkv, qkv_stride, rope_table, rows, q_heads, kv_heads, stride_threshold,
+                                              key_stride, sb, out);
+  };
+  if (head_dim == 64) launch(attention_kernel<64>);
+  else launch(attention_kernel<128>);
   return hipGetLastError();
 }
 
