@@ -1,7 +1,9 @@
 // Dequant + MFMA GEMM for gfx950: Y[M, N] = X[M, K] * W[N, K]^T with W in
 // Q4_K (GGUF blocks) or Q6_K (split layout), X f16, fp32 accumulate.
 //
-// Three kernels share the decode, the epilogues and the split-K contract:
+// The kernels share the decode and the split-K contract:
+//  * gemm_wide_kernel: passes of a few hundred tokens, 64 MI x 128 x 64 tiles,
+//    8 waves, W decoded in the kernel from the tiled copy.
 //  * gemm_kernel<BM>: BM x 128 x 64 tiles (BM 128 or 256), 4 waves, both
 //    operands staged in LDS through registers, W decoded in the kernel.
 //  * gemm_big_kernel: 256 x 256 x 64 tiles, 8 waves of 64 x 128, X copied
@@ -789,6 +791,399 @@ __global__ __launch_bounds__(WM * BN / 128 * 64) void gemm_f16_kernel(const uint
   f16_epilogue<EPI, K16, AI>(acc, m0 + wm * 32 * MI, n0 + wn * 128, lane, M, N, out, ldo, bz);
 }
 
+// ---------------------------------------------------------------------------
+// Passes of a few hundred tokens: BM x 128 tiles (BM = 64 MI), 8 waves (4
+// along M x 2 along N) of 16 MI rows x 64 columns, W decoded in the kernel
+// from the tiled copy. Every weight is decoded once per BM rows, so at these
+// sizes the decode costs less than writing and reading an f16 expansion (four
+// layers of one 500-token request 541 -> 449 us, of 320 tokens 480 -> 397).
+// Bound by the LDS (fragment reads, copies and decoded weights: a step of 128 x
+// 128 x 128 takes 1.3 us, its MFMAs 0.4) and by each step's chain of barrier,
+// fragment reads and MFMAs, which the decode no longer adds to.
+//  * X: stages of BM rows x 64 columns (128 for BM <= 128, half the barriers)
+//    copied global -> LDS (gemm_f16_kernel's layout), in a ring of 3: the copies
+//    of step s + 2 are issued in step s.
+//  * W: wave w loads the raw bytes of tile rows 16w .. +16, 256 columns at a
+//    time (whole lines), two blocks ahead, and decodes 128 columns into one of
+//    two LDS buffers [128 rows][256 B] while the other is in use. With two
+//    steps to a buffer waves 0-3 decode in its first and waves 4-7 in its
+//    second, so of the two waves on a SIMD one decodes while the other issues
+//    MFMAs. 16-byte chunk c of LDS row p sits in slot c ^ (p & 15); the rows are
+//    in f16_w_row<true>'s order, so a lane's accumulators are runs of 8
+//    features of one token.
+// Columns: wave wn owns 32 wn .. +32 and 64 + 32 wn .. +32, the gate and up
+// rows of the same features in the interleaved gate/up layout.
+// ---------------------------------------------------------------------------
+
+// Raw bytes of 16 rows x 256 values from the tiled copy, lane (c, kq) = (row,
+// l / 16); half(h) decodes the lane's 32 values of columns 128 h .. +128: two
+// runs of 16 from 16-byte chunks chunk0() and chunk1() of the 128 columns.
+template <int TYPE>
+struct WideRaw;
+template <>
+struct WideRaw<kQ4_K> {
+  static constexpr int kLoads = 3;
+  u32x4 hdr, q[2];
+  __device__ __forceinline__ void load(const QWeight& w, int tile, int c, int blk, int kq) {
+    const uint8_t* base = w.gv + ((size_t)tile * (w.k >> 8) + blk) * 2304;
+    hdr = *(const u32x4*)(base + 16 * c);
+    q[0] = *(const u32x4*)(base + 256 + 16 * (16 * kq + c));
+    q[1] = *(const u32x4*)(base + 1280 + 16 * (16 * kq + c));
+  }
+  static __device__ __forceinline__ int chunk0(int kq) { return 8 * (kq >> 1) + 2 * (kq & 1); }
+  static __device__ __forceinline__ int chunk1(int kq) { return chunk0(kq) + 4; }
+  template <int H>
+  __device__ __forceinline__ void half(int kq, half8v (&f)[4]) const {
+    float dsc0, ndm0, dsc1, ndm1, lo[16], hi[16];
+    q4k_group_factors(hdr, 2 * H + (kq >> 1), dsc0, ndm0, dsc1, ndm1);
+    const uint32_t words[4] = {q[H].x, q[H].y, q[H].z, q[H].w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      nibbles4_fma(words[i] & 0x0f0f0f0fu, dsc0, ndm0, lo + 4 * i);
+      nibbles4_fma((words[i] >> 4) & 0x0f0f0f0fu, dsc1, ndm1, hi + 4 * i);
+    }
+    f[0] = to_half8(lo), f[1] = to_half8(lo + 8), f[2] = to_half8(hi), f[3] = to_half8(hi + 8);
+  }
+};
+template <>
+struct WideRaw<kQ6_K> {
+  static constexpr int kLoads = 5;
+  // lane kq of a half: quadrants kq & 1 and that + 2, lanes 16 (kq >> 1) .. +16
+  u32x4 ql[2], qh[2], sc;
+  uint16_t d;
+  __device__ __forceinline__ void load(const QWeight& w, int tile, int c, int blk, int kq) {
+    const uint8_t* base = w.gv + ((size_t)tile * (w.k >> 8) + blk) * 3360;
+    const int qa = kq & 1, jh = kq >> 1;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      ql[h] = *(const u32x4*)(base + 1024 * jh + 16 * (16 * (2 * h + qa) + c));
+      qh[h] = *(const u32x4*)(base + 2048 + 512 * jh + 16 * (16 * h + c));
+    }
+    sc = *(const u32x4*)(base + 3072 + 16 * c);
+    d = *(const uint16_t*)(base + 3328 + 2 * c);
+  }
+  static __device__ __forceinline__ int chunk0(int kq) { return 4 * (kq & 1) + 2 * (kq >> 1); }
+  static __device__ __forceinline__ int chunk1(int kq) { return chunk0(kq) + 8; }
+  template <int H>
+  __device__ __forceinline__ void half(int kq, half8v (&f)[4]) const {
+    const int qa = kq & 1, jh = kq >> 1;
+    const uint32_t lw[4] = {ql[H].x, ql[H].y, ql[H].z, ql[H].w}, hw[4] = {qh[H].x, qh[H].y, qh[H].z, qh[H].w};
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      // scale of (half H, lanes 16 jh.., quadrant Q) is scales[8H + jh + 2Q]
+      const int Q = qa + 2 * r, sb = jh + 2 * qa;  // byte sb of word 2H + r
+      const uint32_t sw = H == 0 ? (r == 0 ? sc.x : sc.y) : (r == 0 ? sc.z : sc.w);
+      const float dsc = h2f(d) * (float)(int8_t)((sw >> (8 * sb)) & 0xffu);
+      float v[16];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t q = ((lw[i] >> (4 * r)) & 0x0f0f0f0fu) | (((hw[i] >> (2 * Q)) & 0x03030303u) << 4);
+        bytes4_fma(opaque(q), dsc, -32.0f * dsc, v + 4 * i);
+      }
+      f[2 * r] = to_half8(v), f[2 * r + 1] = to_half8(v + 8);
+    }
+  }
+};
+template <>
+struct WideRaw<kQ4_0> {
+  static constexpr int kLoads = 2;
+  u32x4 q[2];
+  uint16_t d[2];
+  // lane kq of half h: the 32-value block 4h + kq
+  __device__ __forceinline__ void load(const QWeight& w, int tile, int c, int blk, int kq) {
+    const uint8_t* base = w.gv + ((size_t)tile * (w.k >> 8) + blk) * 2304;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int pair = 2 * h + (kq >> 1);
+      q[h] = *(const u32x4*)(base + 1024 * (kq & 1) + 16 * (16 * pair + c));
+      d[h] = *(const uint16_t*)(base + 2048 + 4 * (16 * pair + c) + 2 * (kq & 1));
+    }
+  }
+  static __device__ __forceinline__ int chunk0(int kq) { return 4 * kq; }
+  static __device__ __forceinline__ int chunk1(int kq) { return 4 * kq + 2; }
+  template <int H>
+  __device__ __forceinline__ void half(int, half8v (&f)[4]) const {
+    const uint32_t words[4] = {q[H].x, q[H].y, q[H].z, q[H].w};
+    const float s = h2f(d[H]);
+    float lo[16], hi[16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      nibbles4_fma(words[i] & 0x0f0f0f0fu, s, -8.0f * s, lo + 4 * i);
+      nibbles4_fma((words[i] >> 4) & 0x0f0f0f0fu, s, -8.0f * s, hi + 4 * i);
+    }
+    f[0] = to_half8(lo), f[1] = to_half8(lo + 8), f[2] = to_half8(hi), f[3] = to_half8(hi + 8);
+  }
+};
+
+constexpr int kWideBN = 128, kWideWBuf = kWideBN * 256;  // bytes of a decoded W buffer
+constexpr int wide_steps(int mi) { return mi <= 2 ? 2 : 1; }  // 64-column sub-steps per barrier
+constexpr int wide_lds_bytes(int mi) { return 3 * 64 * mi * 128 * wide_steps(mi) + 2 * kWideWBuf; }
+
+// (x is not __restrict__: the waits count loads in program order, and a
+// restrict read-only pointer's loads may move across the fences below.)
+template <int TYPE, int EPI, int MI>
+__global__ __launch_bounds__(512) void gemm_wide_kernel(const uint16_t* x, int ldx, QWeight w, int M, int kchunk,
+                                                        void* __restrict__ out, int ldo, int ntx, int nty) {
+  constexpr int KS = wide_steps(MI);                          // 64-column sub-steps per step (and barrier)
+  constexpr int BM = 64 * MI, XSUB = BM * 128, XI = MI * KS;  // copy instructions per wave and stage
+  constexpr int XSTAGE = KS * XSUB;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  uint8_t* sX = smem;               // [3][KS][BM rows][128 B]
+  uint8_t* sW = smem + 3 * XSTAGE;  // [2][128 rows][256 B]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 3, wn = wave >> 2;
+  // Each XCD takes a contiguous run of tiles, row tiles of one column panel
+  // side by side: they share its raw weights in the XCD's L2.
+  int bx, by, bz;
+  {
+    const int i = blockIdx.x, ntiles = gridDim.x, q = ntiles >> 3, r = ntiles & 7, xcd = i & 7;
+    const int t = xcd * q + (xcd < r ? xcd : r) + (i >> 3);
+    by = t % nty;
+    bx = t / nty % ntx;
+    bz = t / (nty * ntx);
+  }
+  const int m0 = by * BM, n0 = bx * kWideBN;
+  const int kbeg = bz * kchunk, nblocks = kchunk >> 8, blk0 = kbeg >> 8;
+
+  const uint16_t* xtile = x + (size_t)m0 * ldx + kbeg;
+  int xoff[MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int r = 8 * MI * wave + 8 * i + (lane >> 3);
+    xoff[i] = (min(m0 + r, M - 1) - m0) * ldx + 8 * ((lane & 7) ^ xswz(r));
+  }
+  auto copy = [&](int slot, int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < KS; ++u)
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+        __builtin_amdgcn_global_load_lds((const void*)(xtile + (s * KS + u) * kBK + xoff[i]),
+                                         (lds_void*)(sX + slot * XSTAGE + u * XSUB + (8 * MI * wave + 8 * i) * 128), 16,
+                                         0, 0);
+  };
+
+  // Decode: row c of the wave's 16-row tile is feature 16 wave + c, LDS row p.
+  const int c = lane & 15, kq = lane >> 4;
+  const int wtile = (n0 >> 4) + wave;
+  const int p = 32 * (wave >> 1) + 16 * ((c >> 2) & 1) + 4 * (2 * (wave & 1) + (c >> 3)) + (c & 3);
+  uint8_t* wdst = sW + p * 256;
+  const int ch0 = WideRaw<TYPE>::chunk0(kq), ch1 = WideRaw<TYPE>::chunk1(kq), psw = p & 15;
+  auto put = [&](int buf, const half8v (&f)[4]) {
+    uint8_t* d = wdst + buf * kWideWBuf;
+    *(half8v*)(d + 16 * (ch0 ^ psw)) = f[0];
+    *(half8v*)(d + 16 * ((ch0 + 1) ^ psw)) = f[1];
+    *(half8v*)(d + 16 * (ch1 ^ psw)) = f[2];
+    *(half8v*)(d + 16 * ((ch1 + 1) ^ psw)) = f[3];
+  };
+
+  float4v acc[MI][4];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+  // 64 columns: sub-step u of an X slot, the W buffer's first or second half
+  auto mfma_step = [&](int slot, int u, int buf, int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const uint8_t* xa = sX + slot * XSTAGE + u * XSUB + (wm * 16 * MI + c) * 128 + 16 * ((4 * ks + kq) ^ xswz(c));
+      const uint8_t* wb = sW + buf * kWideWBuf + (32 * wn + c) * 256 + 16 * ((8 * t + 4 * ks + kq) ^ c);
+      half8v af[MI], bf[4];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) af[i] = *(const half8v*)(xa + i * 2048);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bf[j] = *(const half8v*)(wb + (j < 2 ? 16 * j : 64 + 16 * (j - 2)) * 256);
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[j], af[i], acc[i][j], 0, 0, 0);
+    }
+  };
+
+  // The waits count vector loads in program order: neither the optimizer
+  // nor the scheduler may move them across these fences.
+  auto fence = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // The end of a step: the copies of the next one have landed (n newer loads
+  // may be in flight, which __syncthreads would wait for), everyone's LDS
+  // writes are visible.
+  auto sync = [&](auto n) __attribute__((always_inline)) {
+    fence();
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(n)::value));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    fence();
+  };
+  using Copies = std::integral_constant<int, XI>;
+  using Both = std::integral_constant<int, XI + WideRaw<TYPE>::kLoads>;
+  using None = std::integral_constant<int, 0>;
+
+  // Raw bytes of two blocks: the one being decoded and the one after it, whose
+  // loads follow a step's copies and have two more steps to land.
+  WideRaw<TYPE> raw, next;
+  half8v f[4];
+  raw.load(w, wtile, c, blk0, kq);
+  fence();
+  copy(0, 0);
+  copy(1, 1);
+  fence();
+  next.load(w, wtile, c, blk0 + min(1, nblocks - 1), kq);
+  fence();
+  raw.template half<0>(kq, f);
+  put(0, f);
+  sync(None{});
+  int slot = 0;  // of the block's first step
+  auto after = [](int v, int d) { return v + d >= 3 ? v + d - 3 : v + d; };
+  // A decode's values are stored after the step's own fragment reads and MFMAs
+  // in program order, so that the two can overlap.
+  auto block = [&](int B, WideRaw<TYPE>& cur, WideRaw<TYPE>& nxt, auto is_late, auto left) __attribute__((always_inline)) {
+    // LEFT: blocks after this one, 2 for two or more. With fewer no raw bytes
+    // are loaded (nor counted: a load that nothing uses would not be issued).
+    constexpr int LEFT = decltype(left)::value;
+    constexpr bool LATE = decltype(is_late)::value, LAST = LEFT == 0;
+    using Newer = std::conditional_t<LEFT == 2, Both, Copies>;  // after the loads below
+    auto load_after_next = [&]() __attribute__((always_inline)) {
+      if constexpr (LEFT == 2) {
+        cur.load(w, wtile, c, blk0 + min(B + 2, nblocks - 1), kq);
+        fence();
+      }
+    };
+    if constexpr (KS == 2) {
+      // step 2B: buffer 0, the block's second half goes to buffer 1
+      if constexpr (!LAST) copy(after(slot, 2), 2 * B + 2);
+      fence();
+      cur.template half<1>(kq, f);
+      mfma_step(slot, 0, 0, 0);
+      mfma_step(slot, 1, 0, 1);
+      put(1, f);
+      if constexpr (LAST) sync(None{});
+      else sync(Copies{});  // the next block's raw bytes have landed too
+      // step 2B + 1: buffer 1, the next block's first half goes to buffer 0
+      if constexpr (LAST) {
+        mfma_step(after(slot, 1), 0, 1, 0);
+        mfma_step(after(slot, 1), 1, 1, 1);
+      } else {
+        copy(slot, 2 * B + 3);
+        fence();
+        load_after_next();
+        nxt.template half<0>(kq, f);
+        mfma_step(after(slot, 1), 0, 1, 0);
+        mfma_step(after(slot, 1), 1, 1, 1);
+        put(0, f);
+        sync(Newer{});
+        slot = after(slot, 2);
+      }
+    } else {
+      // steps 4B, 4B + 1: buffer 0; the block's second half goes to buffer 1
+      copy(after(slot, 2), 4 * B + 2);
+      fence();
+      if constexpr (!LATE) cur.template half<1>(kq, f);
+      mfma_step(slot, 0, 0, 0);
+      if constexpr (!LATE) put(1, f);
+      // (the late waves' raw loads were issued after the next step's copies)
+      if constexpr (LATE && !LAST) sync(Both{});
+      else sync(Copies{});
+      copy(slot, 4 * B + 3);
+      fence();
+      if constexpr (LATE) cur.template half<1>(kq, f);
+      mfma_step(after(slot, 1), 0, 0, 1);
+      if constexpr (LATE) put(1, f);
+      sync(Copies{});
+      // steps 4B + 2, 4B + 3: buffer 1; the next block's first half goes to buffer 0
+      if constexpr (LAST) {
+        mfma_step(after(slot, 2), 0, 1, 0);
+        sync(None{});
+        mfma_step(slot, 0, 1, 1);
+      } else {
+        copy(after(slot, 1), 4 * B + 4);
+        fence();
+        if constexpr (!LATE) {
+          load_after_next();
+          nxt.template half<0>(kq, f);
+        }
+        mfma_step(after(slot, 2), 0, 1, 0);
+        if constexpr (LATE) {
+          sync(Copies{});
+        } else {
+          put(0, f);
+          sync(Newer{});
+        }
+        copy(after(slot, 2), 4 * B + 5);
+        fence();
+        if constexpr (LATE) {
+          load_after_next();
+          nxt.template half<0>(kq, f);
+        }
+        mfma_step(slot, 0, 1, 1);
+        if constexpr (LATE) put(0, f);
+        sync(Newer{});
+        slot = after(slot, 1);
+      }
+    }
+  };
+  // The two raw blocks change roles from block to block (no register copies,
+  // which would wait for loads in flight).
+  auto loop = [&](auto is_late) __attribute__((always_inline)) {
+    int B = 0;
+    for (; B + 2 < nblocks; B += 2) {
+      block(B, raw, next, is_late, std::integral_constant<int, 2>{});
+      block(B + 1, next, raw, is_late, std::integral_constant<int, 2>{});
+    }
+    if (B + 2 == nblocks) {
+      block(B, raw, next, is_late, std::integral_constant<int, 1>{});
+      block(B + 1, next, raw, is_late, std::integral_constant<int, 0>{});
+    } else {
+      block(B, raw, next, is_late, std::integral_constant<int, 0>{});
+    }
+  };
+  // (the waves of one workgroup meet at the same barriers in either copy)
+  if (KS == 1 && wave >= 4) loop(std::true_type{});
+  else loop(std::false_type{});
+
+  // Lane: token 16i + l%16, features 8(l/16) .. +8 of the wave's two runs of
+  // 32 columns.
+  const int rbase = m0 + wm * 16 * MI + c;
+  const bool vec = (((uintptr_t)out | (uintptr_t)ldo * (EPI == kEpiPartial ? 4 : 2)) & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int row = rbase + 16 * i;
+    if (row >= M) continue;
+#pragma unroll
+    for (int J = 0; J < (EPI == kEpiSwiGLU ? 1 : 2); ++J) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        v[e] = acc[i][2 * J + (e >> 2)][e & 3];
+        if constexpr (EPI == kEpiSwiGLU)
+          v[e] = swiglu((float)(half_t)v[e], (float)(half_t)acc[i][2 + (e >> 2)][e & 3]);
+      }
+      const int col = EPI == kEpiSwiGLU ? (n0 >> 1) + 32 * wn + 8 * kq : n0 + 64 * J + 32 * wn + 8 * kq;
+      const size_t o =
+          ((size_t)(EPI == kEpiPartial || EPI == kEpiPartial16 ? bz * (size_t)M : 0) + row) * ldo + col;
+      if constexpr (EPI == kEpiPartial) {
+        float* y = (float*)out + o;
+        if (vec) {
+          *(float4v*)y = float4v{v[0], v[1], v[2], v[3]};
+          *(float4v*)(y + 4) = float4v{v[4], v[5], v[6], v[7]};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] = v[e];
+        }
+      } else {
+        uint16_t* y = (uint16_t*)out + o;
+        if (vec) {
+          *(half8v*)y = to_half8(v);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] = f2h(v[e]);
+        }
+      }
+    }
+  }
+}
+
 int gemm_splits(const QWeight& w, int m) {
   // Narrow projections (N = hidden) give too few column tiles to fill 256
   // CUs: split K into chunks of at least 1024 columns, at most 4 ways, or 2
@@ -817,7 +1212,23 @@ int mid_splits(const QWeight& w) {
   return s;
 }
 
-enum GemmVariant { kVarBig = 0, kVarLds128 = 1, kVarLds256 = 2, kVarMid = 3 };
+enum GemmVariant { kVarBig = 0, kVarLds128 = 1, kVarLds256 = 2, kVarMid = 3, kVarWide = 4 };
+
+static int wide_tile(const QWeight& w, int m, int splits);
+
+template <int TYPE, int EPI, int MI>
+static void launch_wide(int m, int splits, const uint16_t* x, int ldx, const QWeight& w, int kchunk, void* out, int ldo,
+                        hipStream_t s) {
+  static bool configured = false;  // one attribute call per instantiation
+  if (!configured) {
+    (void)hipFuncSetAttribute((const void*)gemm_wide_kernel<TYPE, EPI, MI>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              wide_lds_bytes(MI));
+    configured = true;
+  }
+  const int ntx = w.n / kWideBN, nty = (m + 64 * MI - 1) / (64 * MI);
+  gemm_wide_kernel<TYPE, EPI, MI><<<ntx * nty * splits, 512, wide_lds_bytes(MI), s>>>(x, ldx, w, m, kchunk, out, ldo,
+                                                                                       ntx, nty);
+}
 
 template <int TYPE, int EPI>
 // Returns whether the launch carried `side` (only the 64-row tiles do).
@@ -832,6 +1243,13 @@ static bool launch_typed(int var, int m, int splits, const uint16_t* x, int ldx,
     }
     dim3 grid((w.n + kBigBN - 1) / kBigBN, (m + kBigBM - 1) / kBigBM, splits);
     gemm_big_kernel<TYPE, EPI><<<grid, 512, kBigLds, s>>>(x, ldx, w, m, kchunk, out, ldo);
+  } else if (var == kVarWide) {
+    switch (wide_tile(w, m, splits)) {
+      case 1: launch_wide<TYPE, EPI, 1>(m, splits, x, ldx, w, kchunk, out, ldo, s); break;
+      case 2: launch_wide<TYPE, EPI, 2>(m, splits, x, ldx, w, kchunk, out, ldo, s); break;
+      case 3: launch_wide<TYPE, EPI, 3>(m, splits, x, ldx, w, kchunk, out, ldo, s); break;
+      default: launch_wide<TYPE, EPI, 4>(m, splits, x, ldx, w, kchunk, out, ldo, s); break;
+    }
   } else if (var == kVarMid && (kchunk / kBK) % kMidDepth == 0) {
     const int ntx = (w.n + 127) / 128, nty = (m + kMidBM - 1) / kMidBM, ntiles = ntx * nty * splits;
     SideExpand e;
@@ -876,6 +1294,33 @@ static bool use_mid(const QWeight& w, int m, int splits) {
   const int wg = ((m + kMidBM - 1) / kMidBM) * ((w.n + 127) / 128) * splits;
   return steps % kMidDepth == 0 && wg <= (w.type == kQ6_K ? 256 : 512);
 }
+
+// Row blocks (MI) of the 64 MI x 128 tiles for this problem, or 0 when it does
+// not take them. Up to max_m tokens they beat both the 64-row tiles and the
+// f16 expansion whatever the shape (2048 columns of K, us: Q4_K 16384 rows at
+// 256, 500 and 1024 tokens 23.7, 35.9, 69.4 against 32.2, 52.4, 71.8 expanded;
+// 3072 rows 18.3, 19.0, 23.9 against 21.9, 22.9 and 31.4; Q4_0 12288 rows at
+// 333 28.4 against 42.9). Beyond, every weight is decoded for 5 or more row
+// tiles and the expansion, done once beside other launches, wins: whole layers
+// of the benchmark's Q4_K / Q6_K weights at 1024, 1152, 1216, 1408 and 1536
+// tokens 14 and 2 us faster, 1 slower, 23 and 24 slower; Q4_0, whose
+// expansions are launches of their own, 18 faster at 1536 and 34 slower at 1920.
+static int wide_tile(const QWeight& w, int m, int splits) {
+  const int max_m = w.type == kQ4_0 ? 1536 : 1152;
+  if (!w.gv || w.n % kWideBN || m <= kGemvMaxM || m > max_m) return 0;
+  // A round of 256 workgroups costs 17.5, 21.5, 28 and 32.5 us at 2048 columns
+  // of K with 1, 2, 3 and 4 row blocks.
+  static const int kRound[4] = {175, 215, 280, 325};
+  int best = 0, cost = 0;
+  for (int mi = 1; mi <= 4; ++mi) {
+    const int wg = ((m + 64 * mi - 1) / (64 * mi)) * (w.n / kWideBN) * splits;
+    const int c = kRound[mi - 1] * ((wg + 255) / 256);
+    if (!best || c < cost) best = mi, cost = c;
+  }
+  return best;
+}
+
+static bool use_wide(const QWeight& w, int m, int splits) { return wide_tile(w, m, splits) > 0; }
 
 // f16 GEMM tile configurations of the two-pass path.
 // kF16T256Tail: 256 x 256 tiles over the rows that fill whole rounds of 256
@@ -1010,11 +1455,11 @@ static int two_pass_tile(const QWeight& w, int m, int splits, bool with_side = f
 // that: its rule in two_pass_tile only picks among two-pass tilings of
 // split problems, which take the two-pass path without it too.
 bool gemm_two_pass(const QWeight& w, int m, int splits) {
-  return !use_mid(w, m, splits) && two_pass_tile(w, m, splits) != kF16None;
+  return !use_wide(w, m, splits) && !use_mid(w, m, splits) && two_pass_tile(w, m, splits) != kF16None;
 }
 
 bool gemm_two_pass_tail(const QWeight& w, int m, int splits) {
-  return !use_mid(w, m, splits) && two_pass_tile(w, m, splits) == kF16T256Tail;
+  return !use_wide(w, m, splits) && !use_mid(w, m, splits) && two_pass_tile(w, m, splits) == kF16T256Tail;
 }
 
 // Operand rows the XCDs' L2s fetch for one tile order: per XCD and round of
@@ -1154,6 +1599,8 @@ static hipError_t launch_fused(const uint16_t* x, int ldx, const QWeight& w, int
   if (epilogue == kEpiSwiGLU && w.n % 128) return hipErrorInvalidValue;
   if (w.type != kQ4_K && w.type != kQ6_K && w.type != kQ4_0) return hipErrorInvalidValue;
   const int kchunk = w.k / splits;
+  // (gemm_wide_kernel addresses a tile's rows by 32-bit element offsets)
+  if (forced < 0 && use_wide(w, m, splits) && (int64_t)256 * ldx <= INT32_MAX) forced = kVarWide;
   if (forced < 0 && use_mid(w, m, splits)) forced = kVarMid;
   const int tile = (wexp && forced < 0) ? two_pass_tile(w, m, splits, side && side->count && side->nblocks > 0)
                                          : kF16None;
