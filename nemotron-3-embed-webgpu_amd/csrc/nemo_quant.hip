@@ -367,38 +367,20 @@ __global__ __launch_bounds__(64 * kGvWaves, PAIR ? 4 : 1) void gemv_kernel(const
   }
 }
 
-// 1024 columns of a row per workgroup, 4 per thread (a division per element, by
-// N in 64 bits, was most of the kernel's time: 96 x 2048 in 4 splits with its GEMV 13.5 -> 13.4 us). VEC:
-// 16-byte loads and 8-byte stores fit.
-template <bool VEC>
-__global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ partials, int splits, int M,
-                                                              int N, uint16_t* __restrict__ y, int ldy, int chunks) {
-  const int m = blockIdx.x / chunks, c = 1024 * (blockIdx.x % chunks) + 4 * threadIdx.x;
-  if (c >= N) return;
-  const float* p = partials + (size_t)m * N + c;
-  uint16_t* o = y + (size_t)m * ldy + c;
-  if constexpr (VEC) {
-    float4v s = {0.f, 0.f, 0.f, 0.f};
-    for (int i = 0; i < splits; ++i) s += *(const float4v*)(p + (size_t)i * M * N);
-    *(half4v*)o = __builtin_convertvector(s, half4v);
-  } else {
-    for (int e = 0; e < 4 && c + e < N; ++e) {
-      float s = 0.f;
-      for (int i = 0; i < splits; ++i) s += p[(size_t)i * M * N + e];
-      o[e] = f2h(s);
-    }
-  }
+__global__ void reduce_partials_kernel(const float* __restrict__ partials, int splits, int M, int N,
+                                       uint16_t* __restrict__ y, int ldy) {
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= (int64_t)M * N) return;
+  float s = 0.f;
+  for (int i = 0; i < splits; ++i) s += partials[(size_t)i * M * N + idx];
+  y[(size_t)(idx / N) * ldy + (idx % N)] = f2h(s);
 }
 
 hipError_t launch_reduce_partials(const float* partials, int splits, int m, int n, uint16_t* y, int ldy,
                                   hipStream_t stream) {
-  if (m <= 0 || n <= 0) return hipSuccess;
-  const int chunks = (n + 1023) / 1024;
-  const unsigned grid = (unsigned)m * chunks;
-  if (n % 4 == 0 && ldy % 4 == 0 && (uintptr_t)y % 8 == 0 && (uintptr_t)partials % 16 == 0)
-    reduce_partials_kernel<true><<<grid, 256, 0, stream>>>(partials, splits, m, n, y, ldy, chunks);
-  else
-    reduce_partials_kernel<false><<<grid, 256, 0, stream>>>(partials, splits, m, n, y, ldy, chunks);
+  const int64_t total = (int64_t)m * n;
+  if (total <= 0) return hipSuccess;
+  reduce_partials_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(partials, splits, m, n, y, ldy);
   return hipGetLastError();
 }
 
