@@ -175,27 +175,10 @@ struct GvQ40 {
   }
 };
 
-typedef __attribute__((address_space(3))) void gv_lds_void;
 enum GvMode { kGvStore = 0, kGvPartial = 1, kGvSwiGLU = 2 };
 
-// PAIR (more workgroups than CUs, several token groups): two workgroups on a
-// CU, which cover each other's waits, so 128 registers: X goes global -> LDS
-// without a group in flight in registers, and the sums of 2 groups (4 of one
-// tile) at a time are added and stored before the next ones start. us,
-// 12288 x 2048 Q4_0 at 32, 64, 96 and 160 tokens: 7.9, 12.0, 15.8, 25.2 with
-// every group's sums and the next group's X in registers, 7.1, 10.3, 13.8, 20.6
-// with PAIR; 16384 x 2048 Q4_K 8.9, 12.9, 17.7, 27.9 and 7.8, 11.5, 15.6, 23.1.
-// One workgroup per CU keeps the registers: 2048 x 8192 Q6_K, 256 workgroups,
-// 96 tokens 13.6 against 14.6.
-// Token groups whose sums are held and added together: at most 8 tile sums, one
-// for each wave.
-constexpr int gv_batch(int tiles, int ng, bool pair) {
-  const int most = pair ? 4 / tiles : 8 / tiles;
-  return ng < most ? ng : most;
-}
-
-template <int TYPE, int MODE, int kGvTiles, bool TILED = false, int NG = 1, bool PAIR = false>
-__global__ __launch_bounds__(64 * kGvWaves, PAIR ? 4 : 1) void gemv_kernel(const uint16_t* __restrict__ x, int ldx, QWeight w, int M,
+template <int TYPE, int MODE, int kGvTiles, bool TILED = false, int NG = 1>
+__global__ __launch_bounds__(64 * kGvWaves) void gemv_kernel(const uint16_t* __restrict__ x, int ldx, QWeight w, int M,
                                                              void* __restrict__ out, int ldo) {
   using Raw = typename std::conditional<TYPE == kQ4_K, GvQ4K,
                                         typename std::conditional<TYPE == kQ6_K, GvQ6K, GvQ40>::type>::type;
@@ -216,26 +199,65 @@ __global__ __launch_bounds__(64 * kGvWaves, PAIR ? 4 : 1) void gemv_kernel(const
   const size_t row_bytes = qweight_row_bytes(TYPE, w.k);
   uint8_t* sx = smem + wave * kGvXSlice;
 
-  // Load i of token group g: rows 2i, 2i + 1 of its 16 x 256 slice; lane l
-  // takes slot l & 31 of row 2i + l / 32 (chunk (l & 31) ^ row). Registers,
-  // then LDS (the compiler orders the wave's own LDS write and reads), or with
-  // PAIR global -> LDS.
-  half8v xs[8];
-  const uint8_t* xb = (const uint8_t*)(x + 256 * blk);  // uniform base, 32-bit lane offsets
-  auto load_x = [&](int g) __attribute__((always_inline)) {
-    const int t0 = lane >> 5, s = lane & 31;
+  float4v acc[NG][kGvTiles];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int t = 2 * i + t0;
-      const uint8_t* src = xb + 2u * (uint32_t)(min(16 * g + t, M - 1) * ldx + 8 * (s ^ t));
-      if constexpr (PAIR) __builtin_amdgcn_global_load_lds((const void*)src, (gv_lds_void*)(sx + 1024 * i), 16, 0, 0);
-      else xs[i] = *(const half8v*)src;
+  for (int g = 0; g < NG; ++g)
+#pragma unroll
+    for (int t = 0; t < kGvTiles; ++t) acc[g][t] = float4v{0.f, 0.f, 0.f, 0.f};
+  if (blk < nblocks) {
+    // Load i of token group g: rows 2i, 2i + 1 of its 16 x 256 slice; lane l
+    // takes slot l & 31 of row 2i + l / 32 (chunk (l & 31) ^ row).
+    // Registers, then LDS: the compiler orders the wave's own LDS write and
+    // reads.
+    half8v xs[8];
+    const uint8_t* xb = (const uint8_t*)(x + 256 * blk);  // uniform base, 32-bit lane offsets
+    auto load_x = [&](int g) {
+      const int t0 = lane >> 5, s = lane & 31;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int t = 2 * i + t0;
+        xs[i] = *(const half8v*)(xb + 2u * (uint32_t)(min(16 * g + t, M - 1) * ldx + 8 * (s ^ t)));
+      }
+    };
+    load_x(0);
+    Raw raw[kGvTiles];
+#pragma unroll
+    for (int t = 0; t < kGvTiles; ++t) {
+      if constexpr (TILED)  // N % 16 == 0: every tile's rows exist
+        raw[t].load_tiled(w, (n0 + 16 * (t % P) + 64 * (t / P)) >> 4, c, blk, kq);
+      else
+        raw[t].load(w, row_bytes, min(n0 + 16 * (t % P) + 64 * (t / P) + c, N - 1), blk, kq);
     }
-  };
-  // GB token groups at a time: their sums are done when the wave's 256 columns
-  // are, and leave the registers before the next ones start.
-  constexpr int GB = gv_batch(kGvTiles, NG, PAIR), BATCHES = (NG + GB - 1) / GB;
-  float4v* red = (float4v*)smem;  // a batch's sums: [wave][group of the batch][tile][lane] at wave * kGvXSlice
+    half8v wf[kGvTiles][8];  // decoded fragments: run r -> 2r, 2r + 1
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) *(half8v*)(sx + 1024 * i + 16 * lane) = xs[i];
+      if (g + 1 < NG) load_x(g + 1);
+      half8v xa[8];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int k = TYPE == kQ4_K ? gv_q4k_run_k(kq, r) : TYPE == kQ6_K ? gv_q6k_run_k(kq, r) : gv_q40_run_k(kq, r);
+        xa[2 * r] = *(const half8v*)(sx + 512 * c + 16 * ((k >> 3) ^ c));
+        xa[2 * r + 1] = *(const half8v*)(sx + 512 * c + 16 * (((k >> 3) + 1) ^ c));
+      }
+      // Tile by tile: the weight loads return in issue order, so the first
+      // tile's decode and MFMAs start while the later tiles' bytes arrive.
+#pragma unroll
+      for (int t = 0; t < kGvTiles; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (g == 0) raw[t].run(kq, r, wf[t][2 * r], wf[t][2 * r + 1]);
+          acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[2 * r], wf[t][2 * r], acc[g][t], 0, 0, 0);
+          acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[2 * r + 1], wf[t][2 * r + 1], acc[g][t], 0, 0, 0);
+        }
+    }
+  }
+  // The 8 waves' sums are added in LDS in rounds of GR token groups (8 tile
+  // sums of 1 KB per wave, in the wave's X region: its fragment reads came
+  // first), each (tile, group) by one wave.
+  constexpr int GR = kGvWaves / kGvTiles, ROUNDS = (NG + GR - 1) / GR;
+  float4v* red = (float4v*)smem;  // round's sums: [wave][group - GR r][tile][lane] at wave * kGvXSlice
   // D layout: lane l, register i -> token 16 g + 4 (l / 16) + i, row l % 16 of the tile.
   auto tile_sum = [&](int pair) {
     float4v s = red[pair * 64 + lane];
@@ -243,35 +265,21 @@ __global__ __launch_bounds__(64 * kGvWaves, PAIR ? 4 : 1) void gemv_kernel(const
     for (int v = 1; v < kGvWaves; ++v) s += red[v * (kGvXSlice / 16) + pair * 64 + lane];
     return s;
   };
-  using Sums = float4v[GB][kGvTiles];
-  auto add = [&](int b, const Sums& acc) __attribute__((always_inline)) {
-    // The 8 waves' sums of the batch are added in LDS in wave order (in each
-    // wave's X region: its fragment reads came first), each (tile, group) by
-    // one wave.
 #pragma unroll
-    for (int gg = 0; gg < GB; ++gg)
+  for (int r = 0; r < ROUNDS; ++r) {
+    if (r > 0) __syncthreads();  // the previous round's sums have been read
 #pragma unroll
-      for (int t = 0; t < kGvTiles; ++t)
-        red[(wave * kGvXSlice / 16) + (gg * kGvTiles + t) * 64 + lane] = acc[gg][t];
+    for (int gg = 0; gg < GR; ++gg)
+      if (GR * r + gg < NG)
+#pragma unroll
+        for (int t = 0; t < kGvTiles; ++t)
+          red[(wave * kGvXSlice / 16) + (gg * kGvTiles + t) * 64 + lane] = acc[min(GR * r + gg, NG - 1)][t];
     __syncthreads();
-    if constexpr (MODE == kGvSwiGLU && PAIR) {
-      // wave -> token 4 (l / 16) + wave % 4 of each lane's 4, group GB b + wave / 4
-      // (a gate and an up float per wave of the workgroup: whole rows of both
-      // would not fit beside the decoded fragments)
-      const int gg = wave >> 2, g = GB * b + gg, m = 16 * g + 4 * kq + (wave & 3);
-      const int f = 64 * (blockIdx.x / G) + 16 * (blockIdx.x % G) + c;
-      if (gg < GB && g < NG && n0 + c + 64 < N) {
-        const float* part = (const float*)smem + 4 * (128 * gg + lane) + (wave & 3);
-        float gs = part[0], us = part[256];
-#pragma unroll
-        for (int v = 1; v < kGvWaves; ++v) gs += part[v * (kGvXSlice / 4)], us += part[v * (kGvXSlice / 4) + 256];
-        if (m < M) ((uint16_t*)out)[(size_t)m * ldo + f] = f2h(swiglu((float)(half_t)gs, (float)(half_t)us));
-      }
-    } else if constexpr (MODE == kGvSwiGLU) {
-      // wave -> gate tile wave % P (and its up tile) of group GB b + wave / P
-      const int tp = wave % P, gg = wave / P, g = GB * b + gg;
+    if constexpr (MODE == kGvSwiGLU) {
+      // wave -> gate tile wave % P (and its up tile) of group GR r + wave / P
+      const int tp = wave % P, gg = wave / P, g = GR * r + gg;
       const int f = 64 * (blockIdx.x / G) + 16 * P * (blockIdx.x % G) + 16 * tp + c;
-      if (gg < GB && g < NG && n0 + 16 * tp + c + 64 < N) {
+      if (gg < GR && g < NG && n0 + 16 * tp + c + 64 < N) {
         const float4v gs = tile_sum(gg * kGvTiles + tp), us = tile_sum(gg * kGvTiles + tp + P);
         uint16_t* y = (uint16_t*)out;
 #pragma unroll
@@ -283,10 +291,10 @@ __global__ __launch_bounds__(64 * kGvWaves, PAIR ? 4 : 1) void gemv_kernel(const
         }
       }
     } else {
-      // wave -> tile wave % T of group GB b + wave / T
-      const int t = wave % kGvTiles, gg = wave / kGvTiles, g = GB * b + gg;
+      // wave -> tile wave % T of group GR r + wave / T
+      const int t = wave % kGvTiles, g = GR * r + wave / kGvTiles;
       const int row = n0 + 16 * (t % P) + 64 * (t / P) + c;
-      if (gg < GB && g < NG && row < N) {
+      if (g < NG && row < N) {
         const float4v s = tile_sum(wave);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -299,71 +307,6 @@ __global__ __launch_bounds__(64 * kGvWaves, PAIR ? 4 : 1) void gemv_kernel(const
         }
       }
     }
-    if (b + 1 < BATCHES) __syncthreads();  // the sums have been read
-  };
-  if (blk >= nblocks) {  // no columns left for this wave
-#pragma unroll
-    for (int b = 0; b < BATCHES; ++b) add(b, Sums{});
-    return;
-  }
-  load_x(0);
-  Raw raw[kGvTiles];
-#pragma unroll
-  for (int t = 0; t < kGvTiles; ++t) {
-    if constexpr (TILED)  // N % 16 == 0: every tile's rows exist
-      raw[t].load_tiled(w, (n0 + 16 * (t % P) + 64 * (t / P)) >> 4, c, blk, kq);
-    else
-      raw[t].load(w, row_bytes, min(n0 + 16 * (t % P) + 64 * (t / P) + c, N - 1), blk, kq);
-  }
-  half8v wf[kGvTiles][8];  // decoded fragments: run r -> 2r, 2r + 1
-  // Group g's 16 tokens, X in the wave's region (`ahead`: group g + 1 follows
-  // in the same batch).
-  auto group = [&](int g, bool ahead, float4v (&acc)[kGvTiles]) __attribute__((always_inline)) {
-    if constexpr (PAIR) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) *(half8v*)(sx + 1024 * i + 16 * lane) = xs[i];
-      if (g + 1 < NG) load_x(g + 1);
-    }
-    half8v xa[8];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int k = TYPE == kQ4_K ? gv_q4k_run_k(kq, r) : TYPE == kQ6_K ? gv_q6k_run_k(kq, r) : gv_q40_run_k(kq, r);
-      xa[2 * r] = *(const half8v*)(sx + 512 * c + 16 * ((k >> 3) ^ c));
-      xa[2 * r + 1] = *(const half8v*)(sx + 512 * c + 16 * (((k >> 3) + 1) ^ c));
-    }
-    if (PAIR && ahead) {  // the region is free once the fragments are in registers
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      load_x(g + 1);
-    }
-    // Tile by tile: the weight loads return in issue order, so the first
-    // tile's decode and MFMAs start while the later tiles' bytes arrive.
-#pragma unroll
-    for (int t = 0; t < kGvTiles; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (g == 0) raw[t].run(kq, r, wf[t][2 * r], wf[t][2 * r + 1]);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[2 * r], wf[t][2 * r], acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[2 * r + 1], wf[t][2 * r + 1], acc[t], 0, 0, 0);
-      }
-  };
-  if constexpr (PAIR) {
-#pragma unroll
-    for (int b = 0; b < BATCHES; ++b) {
-      Sums acc = {};
-      if (b > 0) load_x(GB * b);
-#pragma unroll
-      for (int gg = 0; gg < GB; ++gg)
-        if (GB * b + gg < NG) group(GB * b + gg, gg + 1 < GB && GB * b + gg + 1 < NG, acc[gg]);
-      add(b, acc);
-    }
-  } else {
-    Sums acc[BATCHES] = {};
-#pragma unroll
-    for (int g = 0; g < NG; ++g) group(g, false, acc[g / GB][g % GB]);
-#pragma unroll
-    for (int b = 0; b < BATCHES; ++b) add(b, acc[b]);
   }
 }
 
@@ -432,22 +375,21 @@ template <int TYPE, int MODE, int T, bool TILED>
 static void launch_gemv_groups(dim3 grid, const uint16_t* x, int ldx, const QWeight& w, int m, void* out, int ldo,
                                hipStream_t stream) {
   const int ng = (m + 15) / 16;
-  auto launch = [&](auto kernel) { kernel<<<grid, 64 * kGvWaves, 0, stream>>>(x, ldx, w, m, out, ldo); };
-  auto groups = [&](auto count) {
-    constexpr int NG = decltype(count)::value;
-    if constexpr (T <= 2 && NG > 1) {
-      if (grid.x * grid.y > 256) return launch(gemv_kernel<TYPE, MODE, T, TILED, NG, true>);
-    }
-    launch(gemv_kernel<TYPE, MODE, T, TILED, NG>);
-  };
-  if (ng == 1) groups(std::integral_constant<int, 1>{});
-  else if (ng == 2) groups(std::integral_constant<int, 2>{});
+  if (ng == 1)
+    gemv_kernel<TYPE, MODE, T, TILED, 1><<<grid, 64 * kGvWaves, 0, stream>>>(x, ldx, w, m, out, ldo);
+  else if (ng == 2)
+    gemv_kernel<TYPE, MODE, T, TILED, 2><<<grid, 64 * kGvWaves, 0, stream>>>(x, ldx, w, m, out, ldo);
   else if constexpr (T <= 2) {
-    if (ng == 3) groups(std::integral_constant<int, 3>{});
-    else if (ng == 4) groups(std::integral_constant<int, 4>{});
-    else if (ng <= 6) groups(std::integral_constant<int, 6>{});
-    else if (ng <= 8) groups(std::integral_constant<int, 8>{});
-    else groups(std::integral_constant<int, 10>{});
+    if (ng == 3)
+      gemv_kernel<TYPE, MODE, T, TILED, 3><<<grid, 64 * kGvWaves, 0, stream>>>(x, ldx, w, m, out, ldo);
+    else if (ng == 4)
+      gemv_kernel<TYPE, MODE, T, TILED, 4><<<grid, 64 * kGvWaves, 0, stream>>>(x, ldx, w, m, out, ldo);
+    else if (ng <= 6)
+      gemv_kernel<TYPE, MODE, T, TILED, 6><<<grid, 64 * kGvWaves, 0, stream>>>(x, ldx, w, m, out, ldo);
+    else if (ng <= 8)
+      gemv_kernel<TYPE, MODE, T, TILED, 8><<<grid, 64 * kGvWaves, 0, stream>>>(x, ldx, w, m, out, ldo);
+    else
+      gemv_kernel<TYPE, MODE, T, TILED, 10><<<grid, 64 * kGvWaves, 0, stream>>>(x, ldx, w, m, out, ldo);
   }
 }
 
@@ -456,12 +398,10 @@ static void launch_gemv_kernel(const uint16_t* x, int ldx, const QWeight& w, int
                                hipStream_t stream) {
   const int groups = (w.n + 127) / 128, splits = gemv_splits(w);
   if (w.gv && w.n % 16 == 0) {
-    // Tiled weights: 1 tile per wave while that is at most a workgroup per CU,
-    // 2 beyond (or for SwiGLU): half the X traffic (us on 1 and 2 tiles: Q4_K
-    // 3072 x 2048, 192 or 96 workgroups, 3.5 and 4.2 at 15 tokens, 6.6 and 8.1
-    // at 96; Q4_0 5120 x 2048, 320 or 160, 4.3 and 4.1, 11.0 and 8.4; Q4_0
-    // 2048 x 6144, 384 or 192, 6.8 and 6.5, 13.8 and 11.5).
-    if (MODE == kGvSwiGLU || 8 * groups * splits > 256) {
+    // Tiled weights: 2 tiles per wave when that gives every CU a workgroup
+    // (or for SwiGLU), else 1 (measured on Q4_K: 16384 x 2048 7.7 us on 2
+    // tiles, 7.9 on 4; 2048 x 2048 3.7 us on 1 against 4.5 untiled).
+    if (MODE == kGvSwiGLU || 4 * groups * splits >= 256) {
       launch_gemv_groups<TYPE, MODE, 2, true>(dim3(4 * groups, splits), x, ldx, w, m, out, ldo, stream);
     } else {
       if constexpr (MODE != kGvSwiGLU)
