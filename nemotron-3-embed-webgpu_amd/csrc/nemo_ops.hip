@@ -101,7 +101,9 @@ __device__ __forceinline__ half8v norm_scale8(half8v xv, float inv, const float4
 }
 
 // One row: fetch(c, sum) returns the row's stored values c .. c + 8 and adds
-// the squares of their unrounded forms to `sum`. A row of up to 8 values per
+// the squares of their unrounded forms to `sum`, in order and each with one
+// fmaf: left to contraction, s + v * v may round either product of the first
+// two values, and every later layer of a pass differs with the choice. A row of up to 8 values per
 // thread (hidden 2048 and below) stays in registers between the two passes,
 // its weights loaded beside it; a longer one is read back from x.
 template <typename Fetch>
@@ -143,7 +145,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t* x, const void* _
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float v = (float)xv[i] + dv[i];
-      sum += v * v;  // the unrounded sum, as ops.ts:39-40
+      sum = fmaf(v, v, sum);  // the unrounded sum, as ops.ts:39-40
       stored[i] = (half_t)v;
     }
     *(half8v*)(x + base + c) = stored;
@@ -188,7 +190,7 @@ __global__ __launch_bounds__(256) void embed_norm_kernel(const uint32_t* __restr
     }
     *(half8v*)(xrow + c) = v;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) sum += (float)v[i] * (float)v[i];
+    for (int i = 0; i < 8; ++i) sum = fmaf((float)v[i], (float)v[i], sum);
     return v;
   };
   norm_row(fetch, xrow, w, out + (size_t)t * hidden, hidden, eps, scratch);
