@@ -73,14 +73,39 @@ __device__ __forceinline__ void nibbles4_fma(uint32_t w, float scale, float bias
   out[3] = fmaf(s9, b.y, bias);
 }
 
-// SwiGLU of f16-rounded gate and up values (src/webgpu/ops.ts:85-87) in fp32:
-// g / (1 + e^-g) * u with the hardware exponential and reciprocal (about 1 ulp
-// each; expf and the IEEE division are three times the instructions, and a
-// gate/up tile ends on 64 of these per lane: 384 x 256 tiles 93.7 -> 85.7 us a
-// launch, the 16 x 150 pass 4399 -> 4200). Infinite and NaN gates give what
-// the division gives: e^-g overflows to a reciprocal of 0.
-__device__ __forceinline__ float swiglu(float g, float u) {
-  return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * g)) * u;
+// e^-g for an f16 gate g, the bits of expf(-g): 2^n 2^f with the argument
+// -g log2(e) carried to twice fp32's precision, as expf carries it (one product
+// alone is off by up to 2^-18 at the far gates), but without expf's range
+// checks: past them 2^n overflows or underflows to the same value, and gates
+// above 128, infinity among them, count as 128.
+__device__ __forceinline__ float exp_neg_f16(float g) {
+#pragma clang fp contract(off)  // hi is the rounded product wherever it is used
+  constexpr float kHi = -1.44269504f, kLo = (float)(-1.4426950408889634 - (double)kHi);
+  const float x = fminf(g, 128.0f), hi = x * kHi, n = rintf(hi);
+  return ldexpf(__builtin_amdgcn_exp2f((hi - n) + fmaf(x, kLo, fmaf(x, kHi, -hi))), (int)n);
+}
+
+// f16 of a * b, rounded once (a product rounded to fp32 first differs in one
+// value of 10^4). Written out: left to itself the compiler takes this
+// instruction for single values and the two roundings for vectors of them.
+__device__ __forceinline__ half_t mul_round_f16(float a, float b) {
+  uint32_t r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
+  return __builtin_bit_cast(half_t, (uint16_t)r);
+}
+
+// SwiGLU of f16-rounded gate and up values (src/webgpu/ops.ts:85-87): g / (1 +
+// expf(-g)) in fp32, times u, rounded once to f16. The quotient has the bits
+// of the IEEE division without its range scaling: by a quarter of 1 + e^-g
+// (whose reciprocal stays normal) with the hardware reciprocal and one
+// refinement, four times as large; the fixup gives infinite and NaN operands
+// their quotients. Equal to expf and the division on every f16 gate. 64 of
+// these end a lane's gate/up tile: 16 x 150 tokens 4.31 ms with expf and the
+// division, 4.09 this way.
+__device__ __forceinline__ half_t swiglu(float g, float u) {
+  const float d = fmaf(exp_neg_f16(g), 0.25f, 0.25f);
+  const float r = __builtin_amdgcn_rcpf(d), q = g * r;
+  return mul_round_f16(__builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, g), r, q), d, g), 0.25f * u);
 }
 
 // Round-to-nearest-even f32 -> f16 of eight values (v_cvt_pk_f16_f32 pairs).

@@ -87,7 +87,7 @@ __device__ __forceinline__ void gemm_epilogue(const float16v (&acc)[MI][4], int 
           if (row < M) {
             const float g = (float)(half_t)acc[i][j][r];
             const float u = (float)(half_t)acc[i][j + 2][r];
-            y[(size_t)row * ldo + col] = f2h(swiglu(g, u));
+            y[(size_t)row * ldo + col] = __builtin_bit_cast(uint16_t, swiglu(g, u));
           }
         }
       }
@@ -151,6 +151,7 @@ __device__ __forceinline__ void f16_epilogue(const Acc (&acc)[AI][AJ], int rbase
       for (int c = 0; c < C; ++c) {
         const int at = 32 * J + 16 * c + 8 * (lane / SPAN);
         float v[8];
+        half8v h;
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = value(i, J, c, e);
         if constexpr (EPI == kEpiSwiGLU) {
@@ -158,10 +159,9 @@ __device__ __forceinline__ void f16_epilogue(const Acc (&acc)[AI][AJ], int rbase
           // rows (N % BN == 0). SwiGLU as src/webgpu/ops.ts:85-87 on the
           // f16-rounded gate/up values.
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float g = (float)(half_t)v[e], u = (float)(half_t)value(i, J + 2, c, e);
-            v[e] = swiglu(g, u);
-          }
+          for (int e = 0; e < 8; ++e) h[e] = swiglu((float)(half_t)v[e], (float)(half_t)value(i, J + 2, c, e));
+        } else if constexpr (!F32) {
+          h = to_half8(v);
         }
         const int col = (EPI == kEpiSwiGLU ? cbase >> 1 : cbase) + at;
         const int cols = EPI == kEpiSwiGLU ? N >> 1 : N;
@@ -172,14 +172,14 @@ __device__ __forceinline__ void f16_epilogue(const Acc (&acc)[AI][AJ], int rbase
             *(float4v*)((float*)out + o) = float4v{v[0], v[1], v[2], v[3]};
             *(float4v*)((float*)out + o + 4) = float4v{v[4], v[5], v[6], v[7]};
           } else {
-            *(half8v*)((uint16_t*)out + o) = to_half8(v);
+            *(half8v*)((uint16_t*)out + o) = h;
           }
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e)
             if (col + e < cols) {
               if constexpr (F32) ((float*)out)[o + e] = v[e];
-              else ((uint16_t*)out)[o + e] = f2h(v[e]);
+              else ((half_t*)out)[o + e] = h[e];
             }
         }
         if constexpr (EPI == kEpiSwiGLU) __builtin_amdgcn_sched_barrier(0);  // one run's temporaries at a time
@@ -385,7 +385,7 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(const uint16_t* x, int ld
       if (row < M) {
         const float g = (float)(half_t)acc[0][r];
         const float u = (float)(half_t)acc[1][r];
-        y[(size_t)row * ldo + col] = f2h(swiglu(g, u));
+        y[(size_t)row * ldo + col] = __builtin_bit_cast(uint16_t, swiglu(g, u));
       }
     }
   } else {
@@ -788,7 +788,10 @@ __global__ __launch_bounds__(WM * BN / 128 * 64) void gemm_f16_kernel(const uint
     __syncthreads();
     mfma_step(1);
   }
-  f16_epilogue<EPI, K16, AI>(acc, m0 + wm * 32 * MI, n0 + wn * 128, lane, M, N, out, ldo, bz);
+  // (uniform here: kept in vector registers over the loop, the wave's rows and
+  // columns made the 384 x 256 SwiGLU tile spill 23 of them)
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
+  f16_epilogue<EPI, K16, AI>(acc, m0 + uwave % WM * 32 * MI, n0 + uwave / WM * 128, lane, M, N, out, ldo, bz);
 }
 
 // ---------------------------------------------------------------------------
@@ -1153,12 +1156,14 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint16_t* x, int l
 #pragma unroll
     for (int J = 0; J < (EPI == kEpiSwiGLU ? 1 : 2); ++J) {
       float v[8];
+      half8v h;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         v[e] = acc[i][2 * J + (e >> 2)][e & 3];
         if constexpr (EPI == kEpiSwiGLU)
-          v[e] = swiglu((float)(half_t)v[e], (float)(half_t)acc[i][2 + (e >> 2)][e & 3]);
+          h[e] = swiglu((float)(half_t)v[e], (float)(half_t)acc[i][2 + (e >> 2)][e & 3]);
       }
+      if constexpr (EPI != kEpiSwiGLU && EPI != kEpiPartial) h = to_half8(v);
       const int col = EPI == kEpiSwiGLU ? (n0 >> 1) + 32 * wn + 8 * kq : n0 + 64 * J + 32 * wn + 8 * kq;
       const size_t o =
           ((size_t)(EPI == kEpiPartial || EPI == kEpiPartial16 ? bz * (size_t)M : 0) + row) * ldo + col;
@@ -1172,12 +1177,12 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint16_t* x, int l
           for (int e = 0; e < 8; ++e) y[e] = v[e];
         }
       } else {
-        uint16_t* y = (uint16_t*)out + o;
+        half_t* y = (half_t*)out + o;
         if (vec) {
-          *(half8v*)y = to_half8(v);
+          *(half8v*)y = h;
         } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) y[e] = f2h(v[e]);
+          for (int e = 0; e < 8; ++e) y[e] = h[e];
         }
       }
     }

@@ -785,7 +785,7 @@ __global__ void swiglu_kernel(const uint16_t* __restrict__ gu, int rows, int f, 
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const float gv = (float)g[e];
-    o[e] = (half_t)swiglu(gv, (float)u[e]);
+    o[e] = swiglu(gv, (float)u[e]);
   }
   *(half8v*)(out + i) = o;
 }

@@ -287,7 +287,7 @@ __global__ __launch_bounds__(64 * kGvWaves) void gemv_kernel(const uint16_t* __r
           const int m = 16 * g + 4 * kq + i;
           if (m >= M) continue;
           const float gv = (float)(half_t)gs[i], uv = (float)(half_t)us[i];
-          y[(size_t)m * ldo + f] = f2h(swiglu(gv, uv));
+          y[(size_t)m * ldo + f] = __builtin_bit_cast(uint16_t, swiglu(gv, uv));
         }
       }
     } else {
@@ -347,7 +347,7 @@ __global__ void reduce_swiglu_kernel(const float* __restrict__ partials, int spl
   }
   const float g = (float)(half_t)gs;
   const float u = (float)(half_t)us;
-  y[(size_t)m * ldy + f] = f2h(swiglu(g, u));
+  y[(size_t)m * ldy + f] = __builtin_bit_cast(uint16_t, swiglu(g, u));
 }
 
 hipError_t launch_reduce_swiglu(const float* partials, int splits, int m, int n, uint16_t* y, int ldy,
