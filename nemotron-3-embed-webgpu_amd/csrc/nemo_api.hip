@@ -310,7 +310,7 @@ struct nemo_plan {
   int batch = 0, sequence = 0, merged = 0;
   hipStream_t stream = nullptr;
   std::mutex mu;
-  DevPtr ids, x_full, norm_full, x_red, norm_red, qkv, attn, delta, ffn, out, rope, partials, wexp, pool;
+  DevPtr ids, x_full, norm_full, x_red, norm_red, qkv, attn, delta, ffn, out, rope, partials, wexp;
   size_t wexp_halves = 0;
   // f16 expansions of a layer's gate/up and down weights, written by the QKV
   // and O GEMM launches on the CUs their tiles leave idle (see
@@ -854,7 +854,6 @@ nemo_status nemo_plan_create(nemo_model* model, int32_t batch, int32_t sequence,
     if (dn) p->wexp_dn = dev_alloc(dn * 2, "f16 down expansion");
     p->wexp_gu_halves = gu;
     p->wexp_dn_halves = dn;
-    p->pool = dev_alloc((size_t)batch * pool_pieces(p->merged) * H * 4, "pooling sums");
     p->out = dev_alloc((size_t)batch * H * 4, "embeddings");
     const std::vector<float> table = rope_table(sequence, d.head_dim, d.rope_theta);
     p->rope = dev_alloc(table.size() * 4, "RoPE sin/cos table");
@@ -1140,7 +1139,7 @@ static void enqueue_graph(nemo_plan* p, const uint32_t* d_ids, const Ragged& src
     mark(1, false);
   }
   mark(10, true);
-  hip_check(launch_mean_pool(norm_red, dst, H, (float*)p->pool.get(), d_out, s), "mean pool");
+  hip_check(launch_mean_pool(norm_red, dst, H, d_out, s), "mean pool");
   mark(10, false);
 }
 

@@ -66,9 +66,6 @@ hipError_t launch_merge(const uint16_t* norm, const uint16_t* x, const Ragged& s
                         uint16_t* norm_out, uint16_t* x_out, hipStream_t stream);
 
 // Mean over each request's rows, then L2 normalise; out float [count, hidden].
-// `sums`: room for hidden floats per piece, pool_pieces(rows) of each request.
-int pool_pieces(int rows);
-hipError_t launch_mean_pool(const uint16_t* norm, const Ragged& rows, int hidden, float* sums, float* out,
-                            hipStream_t stream);
+hipError_t launch_mean_pool(const uint16_t* norm, const Ragged& rows, int hidden, float* out, hipStream_t stream);
 
 }  // namespace nemo

@@ -850,85 +850,81 @@ hipError_t launch_merge(const uint16_t* norm, const uint16_t* x, const Ragged& s
 // ---------------------------------------------------------------------------
 // Mean pool + L2 normalise (src/webgpu/ops.ts:596-615), in two kernels so a
 // request is read by many CUs:
-//  * pool_sum_kernel, grid (hidden / 64, pieces): a workgroup sums 64 columns
-//    of one piece of kPoolRows rows of a request; thread (g, p) sums 8 columns
-//    (16-byte loads) of rows p, p + 32, ... in order, and the 32 row phases
-//    are added in phase order.
-//  * pool_norm_kernel, one workgroup per request: adds the pieces' sums in
-//    order, divides by the rows and scales to unit length (no epsilon, as the
-//    reference).
-// Every order depends only on the request's length. With whole requests in one
-// workgroup per 64 columns, 3200 rows (a 5000-token request) took 40 us on 32
-// workgroups; in pieces 5.6.
+//  * pool_mean_kernel, grid (hidden / 32, batch): a workgroup owns 32 columns
+//    of one request; thread (g, p) sums 8 columns (16-byte loads) of rows p,
+//    p + 32, ... in order, and the 32 row phases are added in phase order: an
+//    order that depends only on the request's length. Writes the means.
+//  * pool_norm_kernel, one workgroup per request: scales the means to unit
+//    length (no epsilon, as the reference); thread t adds the squares of
+//    columns t, t + 256, ... in order, each with one fmaf.
+// A thread's rows are a chain of additions, not of loads: 16 rows' loads are
+// issued before the first is added. 3200 rows (a 5000-token request), whose
+// chains are 100 rows long: 37.6 us one load at a time on half as many
+// workgroups, 11.2 this way, bound by the loads' latency. (Sums of 256-row
+// pieces take 5.9, but in another order.)
 // ---------------------------------------------------------------------------
 
-constexpr int kPoolRows = 256;
-
-int pool_pieces(int rows) { return (rows + kPoolRows - 1) / kPoolRows; }
-
-__global__ __launch_bounds__(256) void pool_sum_kernel(const uint16_t* __restrict__ norm, Ragged rows, int hidden,
-                                                       float* __restrict__ sums) {
-  __shared__ float part[32][64];
-  int b = 0, piece = blockIdx.y;
-  for (; b < rows.count; ++b) {
-    const int pieces = (rows.start[b + 1] - rows.start[b] + kPoolRows - 1) / kPoolRows;
-    if (piece < pieces) break;
-    piece -= pieces;
-  }
-  if (b >= rows.count) return;
-  const int c0 = blockIdx.x * 64, r0 = rows.start[b] + piece * kPoolRows;
-  const int n = min(kPoolRows, rows.start[b + 1] - r0);
-  const int g = threadIdx.x & 7, p = threadIdx.x >> 3;
+__global__ __launch_bounds__(128) void pool_mean_kernel(const uint16_t* __restrict__ norm, Ragged rows, int hidden,
+                                                        float* __restrict__ out) {
+  __shared__ float part[32][32];
+  const int b = blockIdx.y, c0 = blockIdx.x * 32;
+  const int r0 = rows.start[b], n = rows.start[b + 1] - r0;
+  const int g = threadIdx.x & 3, p = threadIdx.x >> 2;
+  const uint16_t* column = norm + (size_t)r0 * hidden + c0 + 8 * g;
   float total[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  // Rows p + at + 32 i of `count` phases' rounds; past the request's end the
+  // last row is loaded and zeros are added, which change no sum.
+  auto add = [&](int at, auto count) {
+    constexpr int kRows = decltype(count)::value;
+    half8v v[kRows];
 #pragma unroll
-  for (int i = 0; i < kPoolRows / 32; ++i) {
-    const int r = p + 32 * i;
-    if (r < n) {
-      const half8v v = *(const half8v*)(norm + (size_t)(r0 + r) * hidden + c0 + 8 * g);
+    for (int i = 0; i < kRows; ++i) v[i] = *(const half8v*)(column + (size_t)min(p + at + 32 * i, n - 1) * hidden);
+    __builtin_amdgcn_sched_barrier(0);  // (the scheduler would take them one at a time, to fit more waves)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) total[e] += (float)v[e];
-    }
-  }
+    for (int i = 0; i < kRows; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) total[e] += p + at + 32 * i < n ? (float)v[i][e] : 0.f;
+  };
+  int at = 0;
+  for (; at + 4 * 32 < n; at += 16 * 32) add(at, std::integral_constant<int, 16>{});
+  if (at < n) add(at, std::integral_constant<int, 4>{});
 #pragma unroll
   for (int e = 0; e < 8; ++e) part[p][8 * g + e] = total[e];
   __syncthreads();
-  if (threadIdx.x < 64) {
+  if (threadIdx.x < 32) {
     float sum = part[0][threadIdx.x];
     for (int q = 1; q < 32; ++q) sum += part[q][threadIdx.x];
-    sums[(size_t)blockIdx.y * hidden + c0 + threadIdx.x] = sum;
+    out[(size_t)b * hidden + c0 + threadIdx.x] = sum / (float)n;
   }
 }
 
-__global__ __launch_bounds__(512) void pool_norm_kernel(const float* __restrict__ sums, Ragged rows, int hidden,
-                                                        float* __restrict__ out) {
+__global__ __launch_bounds__(256) void pool_norm_kernel(float* __restrict__ out, int hidden) {
   __shared__ float scratch[16];
-  int first = 0;  // the request's first piece
-  for (int b = 0; b < (int)blockIdx.x; ++b) first += (rows.start[b + 1] - rows.start[b] + kPoolRows - 1) / kPoolRows;
-  const int n = rows.start[blockIdx.x + 1] - rows.start[blockIdx.x];
-  const int pieces = (n + kPoolRows - 1) / kPoolRows;
-  const float* s0 = sums + (size_t)first * hidden;
   float* v = out + (size_t)blockIdx.x * hidden;
   float sq = 0.f;
-  for (int c = threadIdx.x * 4; c < hidden; c += blockDim.x * 4) {
-    float4v a = *(const float4v*)(s0 + c);
-#pragma unroll 8
-    for (int i = 1; i < pieces; ++i) a += *(const float4v*)(s0 + (size_t)i * hidden + c);
-    const float4v mean = a / (float)n;
-    *(float4v*)(v + c) = mean;
-    sq += mean.x * mean.x + mean.y * mean.y + mean.z * mean.z + mean.w * mean.w;
+  float keep[8];  // columns up to 2048 stay in registers
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    keep[i] = c < hidden ? v[c] : 0.f;
   }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) sq = fmaf(keep[i], keep[i], sq);
+  for (int c = threadIdx.x + 2048; c < hidden; c += 256) sq = fmaf(v[c], v[c], sq);
   const float inv = 1.0f / sqrtf(block_sum(sq, scratch));
-  for (int c = threadIdx.x * 4; c < hidden; c += blockDim.x * 4) *(float4v*)(v + c) = *(const float4v*)(v + c) * inv;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    if (c < hidden) v[c] = keep[i] * inv;
+  }
+  for (int c = threadIdx.x + 2048; c < hidden; c += 256) v[c] *= inv;
 }
 
-hipError_t launch_mean_pool(const uint16_t* norm, const Ragged& rows, int hidden, float* sums, float* out,
-                            hipStream_t stream) {
+hipError_t launch_mean_pool(const uint16_t* norm, const Ragged& rows, int hidden, float* out, hipStream_t stream) {
   if (rows.count <= 0) return hipSuccess;
   if (hidden % 64) return hipErrorInvalidValue;
-  int pieces = 0;
-  for (int b = 0; b < rows.count; ++b) pieces += pool_pieces(rows.start[b + 1] - rows.start[b]);
-  pool_sum_kernel<<<dim3(hidden / 64, pieces), 256, 0, stream>>>(norm, rows, hidden, sums);
-  pool_norm_kernel<<<rows.count, 512, 0, stream>>>(sums, rows, hidden, out);
+  pool_mean_kernel<<<dim3(hidden / 32, rows.count), 128, 0, stream>>>(norm, rows, hidden, out);
+  pool_norm_kernel<<<rows.count, 256, 0, stream>>>(out, hidden);
   return hipGetLastError();
 }
 
