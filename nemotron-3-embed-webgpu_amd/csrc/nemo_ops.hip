@@ -103,13 +103,13 @@ __device__ __forceinline__ half8v norm_scale8(half8v xv, float inv, const float4
 // One row: fetch(c, sum) returns the row's stored values c .. c + 8 and adds
 // the squares of their unrounded forms to `sum`, in order and each with one
 // fmaf: left to contraction, s + v * v may round either product of the first
-// two values, and every later layer of a pass differs with the choice. A row of up to 8 values per
-// thread (hidden 2048 and below) stays in registers between the two passes,
-// its weights loaded beside it; a longer one is read back from x.
+// two values, and every later layer of a pass differs with the choice. A row
+// of up to 8 values per thread (hidden 2048 and below) stays in registers
+// between the two passes, its weights loaded beside it; a longer one is read
+// back from xrow, which fetch writes (so xrow is not __restrict__).
 template <typename Fetch>
-__device__ __forceinline__ void norm_row(Fetch&& fetch, const uint16_t* __restrict__ xrow,
-                                         const float* __restrict__ w, uint16_t* __restrict__ orow, int hidden,
-                                         float eps, float* scratch) {
+__device__ __forceinline__ void norm_row(Fetch&& fetch, const uint16_t* xrow, const float* __restrict__ w,
+                                         uint16_t* __restrict__ orow, int hidden, float eps, float* scratch) {
   const int c0 = threadIdx.x * 8, step = blockDim.x * 8;
   float sum = 0.f;
   if (hidden <= step) {
