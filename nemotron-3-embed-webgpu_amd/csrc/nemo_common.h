@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 namespace nemo {
 
 typedef _Float16 half_t;
@@ -44,5 +46,20 @@ __device__ __forceinline__ int ragged_find(const Ragged& r, int t) {
 // operations (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt and lgkmcnt
 // left at their maxima).
 constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
+
+// Lets `Kernel` be launched with up to `bytes` of dynamic LDS on the current
+// device: one attribute call per kernel and device, from any thread. (The
+// kernel is the template's argument, not its type: kernels of one signature
+// have one type, and would share a flag.)
+template <auto Kernel>
+inline void allow_lds(int bytes) {
+  static std::atomic<uint64_t> done{0};  // bit d: device d
+  int device = 0;
+  (void)hipGetDevice(&device);
+  const uint64_t bit = 1ull << (device & 63);
+  if (done.load(std::memory_order_acquire) & bit) return;
+  (void)hipFuncSetAttribute((const void*)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  done.fetch_or(bit, std::memory_order_release);
+}
 
 }  // namespace nemo

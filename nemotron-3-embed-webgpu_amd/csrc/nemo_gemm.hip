@@ -1224,12 +1224,7 @@ static int wide_tile(const QWeight& w, int m, int splits);
 template <int TYPE, int EPI, int MI>
 static void launch_wide(int m, int splits, const uint16_t* x, int ldx, const QWeight& w, int kchunk, void* out, int ldo,
                         hipStream_t s) {
-  static bool configured = false;  // one attribute call per instantiation
-  if (!configured) {
-    (void)hipFuncSetAttribute((const void*)gemm_wide_kernel<TYPE, EPI, MI>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              wide_lds_bytes(MI));
-    configured = true;
-  }
+  allow_lds<gemm_wide_kernel<TYPE, EPI, MI>>(wide_lds_bytes(MI));
   const int ntx = w.n / kWideBN, nty = (m + 64 * MI - 1) / (64 * MI);
   gemm_wide_kernel<TYPE, EPI, MI><<<ntx * nty * splits, 512, wide_lds_bytes(MI), s>>>(x, ldx, w, m, kchunk, out, ldo,
                                                                                        ntx, nty);
@@ -1240,12 +1235,7 @@ template <int TYPE, int EPI>
 static bool launch_typed(int var, int m, int splits, const uint16_t* x, int ldx, const QWeight& w, int kchunk,
                          void* out, int ldo, hipStream_t s, const SideExpand* side) {
   if (var == kVarBig) {
-    static bool configured = false;  // one attribute call per instantiation
-    if (!configured) {
-      (void)hipFuncSetAttribute((const void*)gemm_big_kernel<TYPE, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                kBigLds);
-      configured = true;
-    }
+    allow_lds<gemm_big_kernel<TYPE, EPI>>(kBigLds);
     dim3 grid((w.n + kBigBN - 1) / kBigBN, (m + kBigBM - 1) / kBigBM, splits);
     gemm_big_kernel<TYPE, EPI><<<grid, 512, kBigLds, s>>>(x, ldx, w, m, kchunk, out, ldo);
   } else if (var == kVarWide) {
@@ -1532,20 +1522,17 @@ static void launch_f16(int epilogue, dim3 grid, const uint16_t* x, int ldx, cons
     e = *side;
     nside = (int)std::min<int64_t>(1024, (e.nblocks + threads / 8 - 1) / (threads / 8));
   }
-  auto launch = [&](auto kernel) {
-    static bool configured = false;  // one attribute call per instantiation
-    if (!configured) {
-      (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-      configured = true;
-    }
+  constexpr bool k16 = WM == 4 && MI >= 2;  // 16 x 16 x 32 MFMAs on the 4- and 8-wave tiles of 64+ rows a wave
+  auto launch = [&](auto epi) {
+    constexpr auto kernel = gemm_f16_kernel<decltype(epi)::value, BN, WM, MI, k16>;
+    allow_lds<kernel>(lds);
     kernel<<<ntiles + nside, threads, lds, stream>>>(x, ldx, wexp, w.n, w.k, m, kchunk, out, ldo, (int)grid.x,
                                                       (int)grid.y, ntiles, gw, e);
   };
-  constexpr bool k16 = WM == 4 && MI >= 2;  // 16 x 16 x 32 MFMAs on the 4- and 8-wave tiles of 64+ rows a wave
-  if (epilogue == kEpiStore) launch(gemm_f16_kernel<kEpiStore, BN, WM, MI, k16>);
-  else if (epilogue == kEpiPartial) launch(gemm_f16_kernel<kEpiPartial, BN, WM, MI, k16>);
-  else if (epilogue == kEpiPartial16) launch(gemm_f16_kernel<kEpiPartial16, BN, WM, MI, k16>);
-  else launch(gemm_f16_kernel<kEpiSwiGLU, BN, WM, MI, k16>);
+  if (epilogue == kEpiStore) launch(std::integral_constant<int, kEpiStore>{});
+  else if (epilogue == kEpiPartial) launch(std::integral_constant<int, kEpiPartial>{});
+  else if (epilogue == kEpiPartial16) launch(std::integral_constant<int, kEpiPartial16>{});
+  else launch(std::integral_constant<int, kEpiSwiGLU>{});
 }
 
 static hipError_t launch_two_pass(const uint16_t* x, int ldx, const QWeight& w, int m, int epilogue, int splits,

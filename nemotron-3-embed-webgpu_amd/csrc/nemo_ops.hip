@@ -755,18 +755,14 @@ hipError_t launch_attention(const uint16_t* qkv, int qkv_stride, const float* ro
   const int cap = attn_round_keys(head_dim);
   const int sb = std::min(cap, (longest_keys + kAttnKeys - 1) / kAttnKeys * kAttnKeys);
   const int lds = 2 * (sb * (head_dim + 8) + head_dim * (sb + 8));
-  auto launch = [&](auto kernel) {
-    static bool configured = false;  // one attribute call per instantiation
-    if (!configured) {
-      (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                2 * (cap * (head_dim + 8) + head_dim * (cap + 8)));
-      configured = true;
-    }
+  auto launch = [&](auto hd) {
+    constexpr auto kernel = attention_kernel<decltype(hd)::value>;
+    allow_lds<kernel>(2 * (cap * (head_dim + 8) + head_dim * (cap + 8)));
     kernel<<<grid, 64 * group, lds, stream>>>(qkv, qkv_stride, rope_table, rows, q_heads, kv_heads, stride_threshold,
                                               key_stride, sb, out);
   };
-  if (head_dim == 64) launch(attention_kernel<64>);
-  else launch(attention_kernel<128>);
+  if (head_dim == 64) launch(std::integral_constant<int, 64>{});
+  else launch(std::integral_constant<int, 128>{});
   return hipGetLastError();
 }
 
