@@ -1591,8 +1591,11 @@ static hipError_t launch_fused(const uint16_t* x, int ldx, const QWeight& w, int
   if (epilogue == kEpiSwiGLU && w.n % 128) return hipErrorInvalidValue;
   if (w.type != kQ4_K && w.type != kQ6_K && w.type != kQ4_0) return hipErrorInvalidValue;
   const int kchunk = w.k / splits;
-  // (gemm_wide_kernel addresses a tile's rows by 32-bit element offsets)
-  if (forced < 0 && use_wide(w, m, splits) && (int64_t)256 * ldx <= INT32_MAX) forced = kVarWide;
+  // gemm_wide_kernel addresses a tile's rows by 32-bit element offsets, and
+  // copies X to LDS in 16-byte pieces: rows that do not start on 16 bytes go to
+  // the 64-row tiles, which load them through registers.
+  if (forced < 0 && use_wide(w, m, splits) && (int64_t)256 * ldx <= INT32_MAX && ((uintptr_t)x | 2 * ldx) % 16 == 0)
+    forced = kVarWide;
   if (forced < 0 && use_mid(w, m, splits)) forced = kVarMid;
   const int tile = (wexp && forced < 0) ? two_pass_tile(w, m, splits, side && side->count && side->nblocks > 0)
                                          : kF16None;

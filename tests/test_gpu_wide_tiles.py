@@ -48,3 +48,22 @@ def test_wide_tiles_bit_identical(torch_cuda, type_, m, n, k, shift):
     y = outs[0].cpu().numpy().view(np.float16).reshape(m, n)[:, cols].astype(np.float64)
     want = x16.astype(np.float64) @ w64.T
     assert np.linalg.norm(y - want) <= 2e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("type_,k", [(12, 512), (14, 256), (2, 768)])
+def test_rows_off_16_bytes(torch_cuda, type_, k):
+    """X that starts 2 bytes past alignment takes the 64-row tiles: the same bits."""
+    torch = torch_cuda
+    m, n = 200, 384
+    raw = GEN[type_](407 + type_, n * k // (32 if type_ == 2 else 256))
+    w = rt.QuantWeight(type_, n, k, raw.tobytes())
+    x16 = torch.from_numpy(synth.normal(408, m * k).astype(np.float16).view(np.int16).copy())
+    outs = []
+    for shift in (0, 1):
+        dx = torch.zeros(m * k + 8, dtype=torch.int16, device="cuda")
+        dx[shift:shift + m * k] = x16.cuda()
+        out = torch.full((m, n), 0x7E00, dtype=torch.int16, device="cuda")
+        w.matmul(dx.data_ptr() + 2 * shift, m, out.data_ptr(), _lib.MATMUL_AUTO)
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
