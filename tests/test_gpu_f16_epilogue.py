@@ -33,7 +33,8 @@ def test_two_pass_stores(torch_cuda, m, n, k, shift):
     assert (out[:shift] == 0x1234).all() and (out[shift + m * n:] == 0x1234).all()
 
 
-@pytest.mark.parametrize("n", [12, 200, 700])  # the GEMV, 64-row tiles, f16 tiles
+# the GEMV, fused tiles of 128 and 192 rows, f16 tiles of 384 x 256, and of 256 x 256 with a rest of 128 x 256
+@pytest.mark.parametrize("n", [12, 200, 700, 1200, 2400])
 @pytest.mark.parametrize("scale", [0.01, 4.0, 2500.0])  # gates of about 0.1, 32 and 20000
 def test_swiglu_over_the_gate_range(torch_cuda, n, scale):
     """One layer whose attention adds nothing (zero output projection), so the

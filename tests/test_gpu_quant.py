@@ -224,10 +224,11 @@ def test_two_pass_bit_identical_to_fused(torch_cuda, type_, m, n, k):
     (1536, 2048, 6144),   # 384 x 256 or 192 x 256 tiles
 ])
 def test_mfma_forms_bit_identical_wide_range(torch_cuda, m, n, k):
-    """The f16 GEMM's 16 x 16 x 32 MFMAs and the fused kernels' 32 x 32 x 16
-    round the same f32 sums at the same points: bit-identical results on
-    activations spread over 2^-10 .. 2^6 with random signs (sums that cancel
-    and long carries, where any other rounding order shows)."""
+    """The 16 x 16 x 32 MFMAs (f16 GEMM, and the fused tiles of 161 to 1152
+    rows) and the 32 x 32 x 16 of the other fused kernels round the same f32
+    sums at the same points: bit-identical results on activations spread over
+    2^-10 .. 2^6 with random signs (sums that cancel and long carries, where
+    any other rounding order shows)."""
     torch = torch_cuda
     seed = 9107 + m + n + k
     raw = synth.random_q4k(seed, n * k // 256)
@@ -243,6 +244,9 @@ def test_mfma_forms_bit_identical_wide_range(torch_cuda, m, n, k):
     torch.cuda.synchronize()
     y = two.cpu().numpy().view(np.float16)
     assert np.isfinite(y).all()
+    assert torch.equal(fused, two)
+    w.matmul(dx.data_ptr(), m, fused.data_ptr(), _lib.MATMUL_GEMM_MID)  # 32 x 32 x 16 at every size
+    torch.cuda.synchronize()
     assert torch.equal(fused, two)
 
 

@@ -124,7 +124,7 @@ def test_attention_with_widely_spread_scores(torch_cuda, hd, n):
     the later blocks raise it, which the test first confirms on the oracle's
     own q and k, then checks the attention stage and the embedding against
     the oracle: keys staged all at once (200 tokens at head_dim 64, 100 at
-    128) and in prepared 32-key rounds (300 and 200)."""
+    128) and in rounds of 64 prepared keys (300 and 200)."""
     H, V, F = 256, 300, 512
     Hq, Hkv = (4, 2) if hd == 64 else (2, 1)
     dims = rt.make_dims(hidden=H, q_heads=Hq, kv_heads=Hkv, head_dim=hd, intermediate=F, layers=1, vocab=V,
