@@ -57,9 +57,6 @@ int attention_prep_keys(const Ragged& rows, int stride_threshold, int key_stride
 // prepared).
 constexpr int attn_round_keys(int head_dim) { return 16384 / head_dim; }
 
-// out[t, :F] = f16(silu(g) * u), g = gu[t, :F], u = gu[t, F:2F].
-hipError_t launch_swiglu(const uint16_t* gu, int rows, int f, uint16_t* out, hipStream_t stream);
-
 // Adjacent-state merge of every request from `src` rows to `dst` rows: the
 // normalized stream and, unless `x` is null, the residual stream.
 hipError_t launch_merge(const uint16_t* norm, const uint16_t* x, const Ragged& src, const Ragged& dst, int hidden,

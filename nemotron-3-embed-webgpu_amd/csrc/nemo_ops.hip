@@ -767,33 +767,6 @@ hipError_t launch_attention(const uint16_t* qkv, int qkv_stride, const float* ro
 }
 
 // ---------------------------------------------------------------------------
-// SwiGLU (src/webgpu/ops.ts:74-88).
-// ---------------------------------------------------------------------------
-
-__global__ void swiglu_kernel(const uint16_t* __restrict__ gu, int rows, int f, uint16_t* __restrict__ out) {
-  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
-  const int64_t total = (int64_t)rows * f;
-  if (i >= total) return;
-  const int64_t r = i / f, c = i - r * f;
-  const half8v g = *(const half8v*)(gu + r * 2 * f + c);
-  const half8v u = *(const half8v*)(gu + r * 2 * f + f + c);
-  half8v o;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float gv = (float)g[e];
-    o[e] = swiglu(gv, (float)u[e]);
-  }
-  *(half8v*)(out + i) = o;
-}
-
-hipError_t launch_swiglu(const uint16_t* gu, int rows, int f, uint16_t* out, hipStream_t stream) {
-  const int64_t vec = (int64_t)rows * f / 8;
-  if (vec <= 0) return hipSuccess;
-  swiglu_kernel<<<(unsigned)((vec + 255) / 256), 256, 0, stream>>>(gu, rows, f, out);
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
 // Adjacent-state token merge (src/webgpu/ops.ts:629-660): output position 0
 // is source row 0 (BOS); position p > 0 averages source rows [start, end) with
 // start = 1 + (p-1)(S-1)/(T-1), end = max(1 + p(S-1)/(T-1), start+1) min S.
