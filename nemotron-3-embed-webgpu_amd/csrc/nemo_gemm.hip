@@ -1,5 +1,5 @@
 // Dequant + MFMA GEMM for gfx950: Y[M, N] = X[M, K] * W[N, K]^T with W in
-// Q4_K (GGUF blocks) or Q6_K (split layout), X f16, fp32 accumulate.
+// Q4_K (GGUF blocks), Q6_K or Q4_0 (split layouts), X f16, fp32 accumulate.
 //
 // The kernels share the decode and the split-K contract:
 //  * gemm_wide_kernel: passes of a few hundred tokens, 64 MI x 128 x 64 tiles,
@@ -10,17 +10,20 @@
 //    global -> LDS directly, W decoded in the kernel (Q4_K, large problems).
 //  * expand_kernel + gemm_f16_kernel (two-pass): W expanded to f16 once per
 //    call, then 256 x 256 x 64 tiles with both operands copied global -> LDS.
-// Every wave owns whole 128-column groups, so the gate/up projection finishes
-// SwiGLU in registers: the plan stores gate_up with rows interleaved per
-// 128-row group (64 gate rows, then the matching 64 up rows), and a lane
-// holds g and u of the same (token, feature) in column blocks j and j+2.
+// The gate/up projection finishes SwiGLU in registers: the plan stores gate_up
+// with rows interleaved per 128-row group (64 gate rows, then the matching 64
+// up rows), and every wave owns whole groups, or 32-column runs of the gate
+// rows with the same runs of their up rows, so a lane holds g and u of the
+// same (token, feature).
 //
-// Split-K: blockIdx.z selects a contiguous K range; partial sums are written
-// as fp32 and summed in a fixed order by the consumer (deterministic). The
-// split count depends only on the weight's shape, never on M, and every row's
-// K order is the same in every kernel (sequential 16-column MFMA steps on the
-// same f16 operands), so all paths give identical bits and a
-// token's result does not depend on how many other tokens share the batch.
+// Split-K: each split takes a contiguous K range; partial sums are written as
+// fp32 (or f16, for the plan's residual projections) and summed in a fixed
+// order by the consumer (deterministic). The split count depends on the
+// weight's shape and on whether the pass has kLargeM tokens, and every row's K
+// order is the same in every kernel (MFMA steps in column order on the same
+// f16 operands, whose 16- and 32-column forms give the same bits), so all paths
+// give identical bits and, within a regime of token counts, a token's result
+// does not depend on how many other tokens share the batch.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -122,8 +125,8 @@ __device__ __forceinline__ void gemm_epilogue(const float16v (&acc)[MI][4], int 
 // columns or pointers that 16-byte stores do not fit go value by value. (With
 // X first, a lane held one column of several tokens and stored 2 bytes at a
 // time, 8 times the store instructions: about 8 us of each round of 256 x 256
-// tiles lay outside the K loop. 500-token request, four layers: 577 -> 554 us,
-// 8 x 1500 tokens 5052 -> 4957, 16 x 150 tokens, 16 layers, 4466 -> 4399.)
+// tiles lay outside the K loop. Four layers of 8 x 1500 tokens 5052 -> 4957 us,
+// 16 layers of 16 x 150 4466 -> 4399.)
 template <bool K16>
 __device__ __forceinline__ int f16_w_row(int p) {
   const int low = p & 3, b4 = (p >> 4) & 1, b3 = (p >> 3) & 1, b2 = (p >> 2) & 1;
@@ -629,12 +632,14 @@ __host__ __device__ inline void f16_tile_coords(int i, int ntx, int nty, int nti
 // K16: 16 x 16 x 32 MFMAs (each wave's MI 32-row blocks as 2 MI 16-row
 // blocks, 8 column blocks of 16) instead of 32 x 32 x 16. Every output sums
 // the same f16 products in the same k order, and the two forms give
-// bit-identical results (the fused kernels use 32 x 32 x 16). In the 16 x
-// 150 encoder pass the 16 x 16 form runs the 4- and 8-wave tiles whose waves
-// hold 64 or 96 rows 4-9 % faster (gate/up 256 x 256 137.0 -> 124.5 us, 384 x
-// 256 103.4 -> 99.2, down 256 x 256 61.6 -> 57.5); with 32-row waves
-// (128 x 256) and on the 2-wave 192 x 128 tile it gains nothing or loses up
-// to 1.3 %, and they keep 32 x 32.
+// bit-identical results (gemm_wide_kernel has 16 x 16 x 32 too, the other
+// fused kernels 32 x 32 x 16). In the 16 x 150 encoder pass the 16 x 16 form
+// runs the 4- and 8-wave tiles whose waves hold 64 or 96 rows 4-9 % faster
+// (gate/up 256 x 256 137.0 -> 124.5 us, 384 x 256 103.4 -> 99.2, down 256 x 256
+// 61.6 -> 57.5); with 32-row waves (128 x 256) and on the 2-wave 192 x 128 tile
+// it gains nothing or loses up to 1.3 %, and they keep 32 x 32. Its fragment
+// reads of 16 rows have bank conflicts (19 % of the 256 x 256 gate/up launch's
+// cycles), which the 32-row reads have not.
 template <int EPI, int BN, int WM, int MI, bool K16>
 __global__ __launch_bounds__(WM * BN / 128 * 64) void gemm_f16_kernel(const uint16_t* __restrict__ x, int ldx,
                                                                      const uint16_t* __restrict__ wt, int N, int K,
@@ -799,10 +804,14 @@ __global__ __launch_bounds__(WM * BN / 128 * 64) void gemm_f16_kernel(const uint
 // along M x 2 along N) of 16 MI rows x 64 columns, W decoded in the kernel
 // from the tiled copy. Every weight is decoded once per BM rows, so at these
 // sizes the decode costs less than writing and reading an f16 expansion (four
-// layers of one 500-token request 541 -> 449 us, of 320 tokens 480 -> 397).
-// Bound by the LDS (fragment reads, copies and decoded weights: a step of 128 x
-// 128 x 128 takes 1.3 us, its MFMAs 0.4) and by each step's chain of barrier,
-// fragment reads and MFMAs, which the decode no longer adds to.
+// layers of one 500-token request 526 us without these tiles, 451 with them, of
+// 320 tokens 481 and 398). Bound by each step's chain of barrier, fragment
+// reads and MFMAs with one workgroup on a CU (two waves on a SIMD): at 320 and
+// 500 tokens the MFMAs are busy 6-27 % of the cycles, the LDS 14-32 % and
+// another 4-11 % in bank conflicts, and the projections of fewer than 256
+// workgroups leave CUs idle. Tiles of 256 rows spill 6 (Q4_0) to 41 (Q6_K)
+// registers, mostly in the closing blocks; spilled loads and stores only make
+// the counted waits stricter.
 //  * X: stages of BM rows x 64 columns (128 for BM <= 128, half the barriers)
 //    copied global -> LDS (gemm_f16_kernel's layout), in a ring of 3: the copies
 //    of step s + 2 are issued in step s.
@@ -1291,15 +1300,17 @@ static bool use_mid(const QWeight& w, int m, int splits) {
 }
 
 // Row blocks (MI) of the 64 MI x 128 tiles for this problem, or 0 when it does
-// not take them. Up to max_m tokens they beat both the 64-row tiles and the
-// f16 expansion whatever the shape (2048 columns of K, us: Q4_K 16384 rows at
-// 256, 500 and 1024 tokens 23.7, 35.9, 69.4 against 32.2, 52.4, 71.8 expanded;
-// 3072 rows 18.3, 19.0, 23.9 against 21.9, 22.9 and 31.4; Q4_0 12288 rows at
-// 333 28.4 against 42.9). Beyond, every weight is decoded for 5 or more row
-// tiles and the expansion, done once beside other launches, wins: whole layers
-// of the benchmark's Q4_K / Q6_K weights at 1024, 1152, 1216, 1408 and 1536
-// tokens 14 and 2 us faster, 1 slower, 23 and 24 slower; Q4_0, whose
-// expansions are launches of their own, 18 faster at 1536 and 34 slower at 1920.
+// not take them. Up to max_m tokens they beat the 64-row tiles and the f16
+// expansion on the matrices measured (2048 columns of K, us: Q4_K 16384 rows at
+// 256, 500 and 1024 tokens 23.1, 36.8, 71.2 against 30.8, 52.8, 73.4; 3072 rows
+// 17.9, 18.1, 23.0 against 21.2, 21.8 and 29.1; Q4_0 12288 rows at 333 28.5
+// against 44.5). The bound is that of whole layers, whose expansions are done
+// once beside other launches: of Q4_K / Q6_K weights at hidden 2048 and FFN
+// 8192, at 1024, 1152, 1216, 1408 and 1536 tokens 14 and 2 us faster, 1 slower,
+// 23 and 24 slower; of Q4_0, whose expansions are launches of their own, 18
+// faster at 1536 and 34 slower at 1920. Single matrices cross elsewhere: at
+// 1536 tokens 3072 rows still take 28.4 us against 41.0, 16384 rows 103.2
+// against 99.1.
 static int wide_tile(const QWeight& w, int m, int splits) {
   const int max_m = w.type == kQ4_0 ? 1536 : 1152;
   if (!w.gv || w.n % kWideBN || m <= kGemvMaxM || m > max_m) return 0;

@@ -604,13 +604,15 @@ __global__ __launch_bounds__(512) void attention_kernel(const uint16_t* __restri
 // flight under round r. The two blocks' score chains are independent, and one
 // block's exponentials run under the other's MFMAs.
 //
-// Bound by the LDS reads (1 KB per MFMA, as long as the MFMA takes on four
-// SIMDs) and the exponentials together. What it replaced staged 32 keys per
-// barrier through registers for one workgroup of `group` waves (3 at the
-// published heads: 6 waves on a CU, on 2 of its SIMDs 2): 8 x 1500 tokens,
-// 24 heads of 128, 458 -> 277 us a layer; 5000 tokens, 32 heads of 64, every
-// third key, 109 -> 101, 3200 64 -> 53 (same bits). The KV head runs fastest in the grid, so with 8 of
-// them each XCD's L2 holds the images of one.
+// Bound by the vector ALU (exponentials, maxima and conversions; active 62 % of
+// the cycles at 5000 tokens and 32 heads of 64) and the MFMAs (31 %), which
+// take turns on a SIMD of few waves; the LDS is active 16 %, without
+// conflicts. What it replaced staged 32 keys per barrier through registers for
+// one workgroup of `group` waves (3 at 24 heads of 128: 6 waves on a CU, on 2
+// of its SIMDs 2): 8 x 1500 tokens, 24 heads of 128, 458 -> 277 us a layer; 5000
+// tokens, 32 heads of 64, every third key, 109 -> 101, 3200 64 -> 53 (same
+// bits). The KV head runs fastest in the grid, so with 8 of them each XCD's L2
+// holds the images of one.
 template <int HD>
 __global__ __launch_bounds__(256, HD == 128 ? 2 : 4)
 void attention_long_kernel(const uint16_t* __restrict__ qkv, int qkv_stride, const float* __restrict__ table,
